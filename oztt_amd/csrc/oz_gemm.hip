@@ -30,18 +30,12 @@
 //     power, down; the matrix cores are power-limited, so that raises their clock.
 #include "oz2_modular.hpp"
 #include "oz_gemm_common.hpp"
-#include "oz_internal.hpp"
+#include "oz_gemm_launch.hpp"
+#include "oz_gemm_tiles.hpp"
 
 namespace {
 
 using namespace ozg;
-
-// Output modes. PRODUCTS: C[b] = A[b] Bt[b]^T as int32. DIGITS: the same products reduced in the
-// epilogue to the CRT digit for modulus b ((C mod m_b) y_b mod m_b, from dc.m/y[b]; a digit 0 may be
-// stored as m_b, oz2::mod_mul_f64), C as uint8. DIAG
-// (scheme I): C[d] = sum_{i <= d} A[i] Bt[d-i]^T as int32 for the diagonals d < nbatch, the d+1
-// slice pairs concatenated along K in one accumulation.
-enum GemmMode { PRODUCTS = 0, DIGITS = 1, DIAG = 2 };
 
 constexpr int LOADS = LOADS_A + LOADS_B;  // global->LDS loads per wave per K step
 
@@ -353,6 +347,17 @@ const char* check_gemm(const int8_t* A, const int8_t* Bt, const void* C, int M, 
 template <int MODE>
 int launch_gemm(oz_dev* dev, const int8_t* A, const int8_t* Bt, void* C, int M, int N, int K, int batch, int ldc,
                 long long strideA, long long strideB, long long strideC, const oz2::DigitConsts& dc) {
+    // few tiles, short K or unevenly filled rounds go to the smaller tiles
+    if constexpr (MODE != PRODUCTS) {
+        const oz::ProductArgs args{A, Bt, C, M, N, K, batch, ldc, strideA, strideB, strideC, dc};
+        if constexpr (MODE == DIGITS) {
+            const oz::DigitTile t = oz::digit_tile(dev->cus, M, N, K, batch);
+            if (t != oz::DigitTile::Tile256) return oz::launch_digit_tile(dev, t, args);
+        } else {
+            const oz::DiagTile t = oz::diag_tile(dev->cus, M, N, K, batch);
+            if (t != oz::DiagTile::Tile256) return oz::launch_diag_tile(dev, t, args);
+        }
+    }
     const int tiles_m = M / BM, tiles_n = N / BN;
     const long long tiles = (long long)tiles_m * tiles_n * batch;
     // 1/8 more workgroups than tiles (at least one more per XCD): the XCDs that run ahead take more of
