@@ -39,6 +39,7 @@ HIP_SOURCES = {
     "oz_gemm.hip": [],
     "oz_gemm_tiles.hip": [],
     "oz2_crt.hip": [],
+    "oz2_gemm_crt.hip": [],
     "oz1_slice.hip": ["-fgpu-flush-denormals-to-zero"],
     "oz1_recon.hip": ["-fgpu-flush-denormals-to-zero"],
     "oz2_digits.hip": ["-fgpu-flush-denormals-to-zero"],

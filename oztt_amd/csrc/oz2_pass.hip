@@ -15,6 +15,8 @@
 // the splitter writes the padding as zeros). Each region starts on a 256-byte boundary.
 #include "oz2_pass.hpp"
 
+#include "oz2_gemm_crt.hpp"
+
 namespace oz2pass {
 
 namespace {
@@ -55,6 +57,17 @@ const char* check_plan(const oz2_moduli_dev* mo, const oz2_crt_dev* crt, int Kg)
     return nullptr;
 }
 
+// Products and reconstruction in one kernel (oz2_gemm_crt.hip), without the digits in memory: for short K
+// and at least two 64 x 64 tiles per CU. The whole pass with digits -> fused, us:
+//   4096 x 4096: 211 -> 147 (K 64), 222 -> 173 (128), 266 -> 226 (256), 350 against 333 (512, where the
+//   8192 x 8192 result takes 1241 against 1290); 2048 x 2048: 78 -> 64 (128), 86 -> 78 (256), 104 against
+//   107 (512); 1024 x 1024 (one tile per CU): 38 -> 36 (64), 41 against 44 (256).
+static bool fused_reconstruction(const oz_dev* dev, int M, int N, int Kg, const oz2_crt_dev* crt) {
+    const long long tiles = ((M + 63ll) / 64) * ((N + 63ll) / 64);
+    int width, limbs;
+    return Kg <= 256 && tiles >= 2ll * dev->cus && tiles <= 0x7FFFFFFFll && oz::fused_limbs(crt, Kg, &width, &limbs);
+}
+
 int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, double* C, int ldc, int M, int N, int K,
              const oz2_moduli_dev* mo, const oz2_crt_dev* crt, uint32_t* flags, uint8_t* work, const PassLayout& L) {
     const int S = mo->S;
@@ -68,7 +81,10 @@ int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, do
     // Scheme II rounds the BF16 of the maxima up (reference ozaki2.cpp:143-146)
     if (int st = oz_scale_pair_f64(dev, A, M, K, lda, B, N, ldb, 1, crt->shift, dA, dB, flags, nullptr)) return st;
     if (int st = oz2_split_pair_int8(dev, A, M, K, lda, dA, B, N, ldb, dB, mo, pA, pB, L.Mg, L.Ng, L.Kg)) return st;
-    if (int st = oz2_gemm_digits(dev, pA, pB, dg, L.Mg, L.Ng, L.Kg, S, L.Ng, sA, (long long)L.Ng * L.Kg, sD, crt))
+    const long long sB = (long long)L.Ng * L.Kg;
+    if (fused_reconstruction(dev, M, N, L.Kg, crt))
+        return oz::launch_fused(dev, oz::FusedArgs{pA, pB, M, N, L.Kg, sA, sB, crt, dA, dB, C, ldc});
+    if (int st = oz2_gemm_digits(dev, pA, pB, dg, L.Mg, L.Ng, L.Kg, S, L.Ng, sA, sB, sD, crt))
         return st;
     return oz2_crt_digits_f64(dev, dg, M, N, L.Ng, sD, crt, dA, dB, C, ldc);
 }
