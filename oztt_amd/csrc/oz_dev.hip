@@ -57,8 +57,8 @@ int oz_dev_open(int device_id, oz_dev** out) {
         }
     }
     if (hipDeviceGetAttribute(&d->cus, hipDeviceAttributeMultiprocessorCount, device_id) != hipSuccess ||
-        hipMalloc(&d->queue, 16 * sizeof(int)) != hipSuccess ||
-        hipMemsetAsync(d->queue, 0, 16 * sizeof(int), d->stream) != hipSuccess) {  // ordered before every launch
+        hipMalloc(&d->queue, oz_dev::kQueueInts * sizeof(int)) != hipSuccess ||
+        hipMemsetAsync(d->queue, 0, oz_dev::kQueueInts * sizeof(int), d->stream) != hipSuccess) {  // ordered before every launch
         oz_dev_close(d);
         return OZ_ERR_HIP;
     }

@@ -15,7 +15,12 @@ struct oz_dev {
     hipStream_t stream = nullptr;
     hipEvent_t events[OZ_EVENT_SLOTS] = {};
     std::string error;
-    int* queue = nullptr;   // tile pool counters of the INT8 product kernel (16 ints, zero between launches)
+    // Device words of the handle, zero between launches (passes, for the range flags): tile pool counters of
+    // the INT8 product kernel (queue[0..1]), the range flags of the whole pass (kPassFlags, two words), and
+    // for the scale's chunked column strips their arrival counters (kStripCounts) and maxima (kStripKeys).
+    int* queue = nullptr;
+    static constexpr int kPassFlags = 8, kStripCounts = 16, kStrips = 128, kStripKeys = kStripCounts + kStrips,
+                         kQueueInts = kStripKeys + 32 * kStrips;
     int cus = 0;            // compute units: a product launch of at most this many tiles needs no pool
     // oz_time_products_begin: event slots of the product launches to time (-1: none), and whether
     // one has run under the request
