@@ -36,6 +36,7 @@ HIP_SOURCES = {
     "oz_dev.hip": [],
     "oz_scale.hip": [],
     "oz2_split.hip": ["-fgpu-flush-denormals-to-zero", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "oz2_prep.hip": ["-fgpu-flush-denormals-to-zero", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "oz_gemm.hip": [],
     "oz_gemm_tiles.hip": [],
     "oz2_crt.hip": [],

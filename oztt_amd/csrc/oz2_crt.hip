@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "oz2_gemm_crt.hpp"
 #include "oz2_modular.hpp"
 #include "oz_internal.hpp"
 
@@ -274,55 +275,85 @@ __global__ void __launch_bounds__(256) crt_kernel(const int32_t* __restrict__ C,
 }
 
 // From the CRT digits k_s (uint8, written by the product kernel, k_s <= m_s <= 255): one thread per 4
-// consecutive output elements of a row, so that each plane read is one 32-bit word per thread.
+// consecutive output elements of a row, so that each plane read is one 32-bit word per thread (or per
+// element, below).
 // Limbs of 40 bits: every k_s Q_s,l < 2^48 and every sum over at most 24 moduli stays below 2^53, so
 // 4 limbs cover the C3 plan (S M < 2^139) where 32-bit limbs need 5. A digit enters its FMAs as the
 // FP64 denormal k 2^-1074 (its byte in the low word, zero above: one bit-field extract, no
 // conversion), against limbs of Q_s stored times 2^984, so the accumulators hold V 2^-90 exactly
 // (integers times 2^-90 below 2^-37: normal doubles).
-template <int L>
+// V elements per thread: 4 (one row per blockIdx.y) for large results; 1, with the elements of all rows
+// numbered through, for small ones, which are bound by the latency of one thread's chain (about 200 FP64
+// operations per element) and would leave most lanes idle: 8.8 -> 7.0 us at 256 x 256.
+// move_flags: thread 0 and 1 of the first workgroup move the range flags of a whole pass (run_pass) from
+// fsrc to fdst and zero fsrc for the next pass.
+__device__ __forceinline__ void move_flags(uint32_t* __restrict__ fsrc, uint32_t* __restrict__ fdst) {
+    if (fdst && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2) {
+        fdst[threadIdx.x] = fsrc[threadIdx.x];
+        fsrc[threadIdx.x] = 0u;
+    }
+}
+
+template <int V>
+struct DigitWord;
+template <>
+struct DigitWord<1> {
+    using type = uint8_t;
+};
+template <>
+struct DigitWord<4> {
+    using type = uint32_t;
+};
+
+template <int L, int V>
 __global__ void __launch_bounds__(256) crt_digits_kernel(const uint8_t* __restrict__ D, int M, int N, int ldd,
                                                          long long sD, CrtLimbs40 a, const int32_t* __restrict__ dA,
                                                          const int32_t* __restrict__ dB, double* __restrict__ out,
-                                                         int ldo) {
-    const int j0 = 4 * (blockIdx.x * 256 + threadIdx.x);
-    const int i = blockIdx.y;
-    if (j0 >= N) return;
-    const uint32_t* d = reinterpret_cast<const uint32_t*>(D + (long long)i * ldd + j0);
-    const long long sw = sD / 4;
+                                                         int ldo, uint32_t* __restrict__ fsrc,
+                                                         uint32_t* __restrict__ fdst) {
+    using Word = typename DigitWord<V>::type;
+    move_flags(fsrc, fdst);
+    const int x0 = blockIdx.x * 256 + threadIdx.x;
+    const int i = V == 1 ? x0 / N : (int)blockIdx.y;
+    const int j0 = V == 1 ? x0 - i * N : V * x0;
+    if (V == 1 ? i >= M : j0 >= N) return;
+    const Word* d = reinterpret_cast<const Word*>(D + (long long)i * ldd + j0);
+    const long long sw = sD / V;
     // every plane's word is requested before the first is used (the planes past S read plane S-1
     // again, so that no load waits on a branch)
     uint32_t v[OZ2_MAXS];
 #pragma unroll
     for (int s = 0; s < OZ2_MAXS; s++) v[s] = d[(long long)min(s, a.S - 1) * sw];
-    double x[4][L];
+    double x[V][L];
 #pragma unroll
-    for (int e = 0; e < 4; e++)
+    for (int e = 0; e < V; e++)
 #pragma unroll
         for (int l = 0; l < L; l++) x[e][l] = 0.0;
 #pragma unroll
     for (int s = 0; s < OZ2_MAXS; s++)
         if (s < a.S) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
+            for (int e = 0; e < V; e++) {
                 const double k = __hiloint2double(0, (int)((v[s] >> (8 * e)) & 0xFFu));  // k 2^-1074
 #pragma unroll
                 for (int l = 0; l < L; l++) x[e][l] = __builtin_fma(k, a.Q[s][l], x[e][l]);
             }
         }
     const int gi = 2 * a.shift - dA[i] - 2 * a.b;
-    double r[4];
+    double r[V];
 #pragma unroll
-    for (int e = 0; e < 4; e++) r[e] = j0 + e < N ? crt_finish<L>(x[e], a, gi - dB[j0 + e]) : 0.0;
+    for (int e = 0; e < V; e++) r[e] = j0 + e < N ? crt_finish<L>(x[e], a, gi - dB[j0 + e]) : 0.0;
     double* o = out + (long long)i * ldo + j0;
-    if (j0 + 3 < N && !(reinterpret_cast<uintptr_t>(o) & 15)) {
+    if constexpr (V == 1) {
+        *o = r[0];
+    } else if (j0 + 3 < N && !(reinterpret_cast<uintptr_t>(o) & 15)) {
         // non-temporal: C (512 MB at C3) is not read again by the pass (0.418 against 0.431 ms)
         typedef double f64x2 __attribute__((ext_vector_type(2)));
         __builtin_nontemporal_store(f64x2{r[0], r[1]}, reinterpret_cast<f64x2*>(o));
         __builtin_nontemporal_store(f64x2{r[2], r[3]}, reinterpret_cast<f64x2*>(o) + 1);
     } else {
 #pragma unroll
-        for (int e = 0; e < 4; e++)
+        for (int e = 0; e < V; e++)
             if (j0 + e < N) o[e] = r[e];
     }
 }
@@ -493,9 +524,13 @@ int crt_limbs40(const CrtLimbs& a, CrtLimbs40& b) {
 
 template <int L>
 int launch_crt_digits(oz_dev* dev, const uint8_t* D, int M, int N, int ldd, long long sD, const CrtLimbs40& a,
-                      const int32_t* dA, const int32_t* dB, double* out, int ldo) {
-    hipLaunchKernelGGL(crt_digits_kernel<L>, dim3(oz::ceil_div(N, 1024), M), dim3(256), 0, dev->stream, D, M, N, ldd,
-                       sD, a, dA, dB, out, ldo);
+                      const int32_t* dA, const int32_t* dB, double* out, int ldo, uint32_t* fsrc, uint32_t* fdst) {
+    if ((long long)M * N <= 1024ll * dev->cus)  // one element per thread: at most 4 waves per SIMD
+        hipLaunchKernelGGL((crt_digits_kernel<L, 1>), dim3(oz::ceil_div((long long)M * N, 256)), dim3(256), 0, dev->stream, D,
+                           M, N, ldd, sD, a, dA, dB, out, ldo, fsrc, fdst);
+    else
+        hipLaunchKernelGGL((crt_digits_kernel<L, 4>), dim3(oz::ceil_div(N, 1024), M), dim3(256), 0, dev->stream, D, M, N, ldd,
+                           sD, a, dA, dB, out, ldo, fsrc, fdst);
     return oz::launch_check(dev, "crt_digits_kernel");
 }
 
@@ -503,7 +538,8 @@ int launch_crt_digits(oz_dev* dev, const uint8_t* D, int M, int N, int ldd, long
 // strides) or uint16 terms (kind 2, element strides); rows go on the grid's y (at most 65535 per
 // launch), so the launch is split in row chunks.
 int crt_launch(oz_dev* dev, const void* C, int kind, int M, int N, int ldc, long long strideC, int nw,
-               const CrtLimbs& a, const int32_t* dA, const int32_t* dB, double* out, int ldo) {
+               const CrtLimbs& a, const int32_t* dA, const int32_t* dB, double* out, int ldo, uint32_t* fsrc = nullptr,
+               uint32_t* fdst = nullptr) {
     const size_t esz = kind == 1 ? 1 : kind == 2 ? 2 : 4;
     if (kind == 1) {
         CrtLimbs40 b;
@@ -514,12 +550,13 @@ int crt_launch(oz_dev* dev, const void* C, int kind, int M, int N, int ldc, long
             double* oi = out + (long long)i0 * ldo;
             int st;
             switch (L) {
-            case 2: st = launch_crt_digits<2>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo); break;
-            case 3: st = launch_crt_digits<3>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo); break;
-            case 4: st = launch_crt_digits<4>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo); break;
-            default: st = launch_crt_digits<5>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo); break;
+            case 2: st = launch_crt_digits<2>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst); break;
+            case 3: st = launch_crt_digits<3>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst); break;
+            case 4: st = launch_crt_digits<4>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst); break;
+            default: st = launch_crt_digits<5>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst); break;
             }
             if (st) return st;
+            fdst = nullptr;  // moved by the first launch
         }
         return OZ_OK;
     }
@@ -542,17 +579,24 @@ int crt_launch(oz_dev* dev, const void* C, int kind, int M, int N, int ldc, long
 }
 
 int crt_f64(oz_dev* dev, const char* name, const void* C, bool digits, int M, int N, int ldc, long long strideC,
-            const oz2_crt_dev* crt, const int32_t* dA, const int32_t* dB, double* out, int ldo) {
+            const oz2_crt_dev* crt, const int32_t* dA, const int32_t* dB, double* out, int ldo, uint32_t* fsrc = nullptr,
+            uint32_t* fdst = nullptr) {
     if (int st = oz::use(dev)) return st;
     if (!C || !crt || !dA || !dB || !out || M <= 0 || N <= 0 || ldc < N || ldo < N || crt->S < 1 ||
         crt->S > OZ2_MAXS || crt->nw < 3 || crt->nw > 8 || (digits && (ldc % 4 || strideC % 4 || ((uintptr_t)C & 3))))
         return oz::fail(dev, OZ_ERR_ARG, "%s: invalid arguments", name);
     CrtLimbs a;
     if (int st = crt_limbs(dev, name, crt, 255u, a)) return st;
-    return crt_launch(dev, C, digits ? 1 : 0, M, N, ldc, strideC, crt->nw, a, dA, dB, out, ldo);
+    return crt_launch(dev, C, digits ? 1 : 0, M, N, ldc, strideC, crt->nw, a, dA, dB, out, ldo, fsrc, fdst);
 }
 
 }  // namespace
+
+int oz::crt_digits_moving_flags(oz_dev* dev, const uint8_t* D, int M, int N, int ldd, long long strideD,
+                                const oz2_crt_dev* crt, const int32_t* dA, const int32_t* dB, double* out, int ldo,
+                                uint32_t* fsrc, uint32_t* fdst) {
+    return crt_f64(dev, "oz2_crt_digits_f64", D, true, M, N, ldd, strideD, crt, dA, dB, out, ldo, fsrc, fdst);
+}
 
 extern "C" int oz2_crt_f64(oz_dev* dev, const int32_t* C, int M, int N, int ldc, long long strideC,
                            const oz2_crt_dev* crt, const int32_t* dA, const int32_t* dB, double* out, int ldo) {

@@ -142,7 +142,11 @@ template <int L>
 __global__ void __launch_bounds__(256, 2) gemm_crt_kernel(
     const int8_t* __restrict__ A, const int8_t* __restrict__ Bt, int K, long long sA, long long sB, int tiles_m,
     int tiles_n, FusedCrt<L> a, const int32_t* __restrict__ dA, const int32_t* __restrict__ dB, int M, int N,
-    double* __restrict__ out, int ldo) {
+    double* __restrict__ out, int ldo, uint32_t* __restrict__ fsrc, uint32_t* __restrict__ fdst) {
+    if (blockIdx.x == 0 && threadIdx.x < 2) {  // the pass's range flags (crt_digits_kernel's move_flags)
+        fdst[threadIdx.x] = fsrc[threadIdx.x];
+        fsrc[threadIdx.x] = 0u;
+    }
     constexpr int TI = 2, TJ = 2, NSTG = 6;
     constexpr int BA = 2 * TI, BB = 2 * TJ;  // 1 KB blocks of a stage
     constexpr int TM = 16 * BA, TN = 16 * BB;
@@ -359,7 +363,7 @@ int launch(oz_dev* dev, const oz::FusedArgs& f, int w) {
     constants<L>(f.crt, w, a);
     const int tm = (f.M + 63) / 64, tn = (f.N + 63) / 64;
     oz::launch_product(dev, gemm_crt_kernel<L>, dim3((unsigned)(tm * tn)), dim3(256), f.A, f.Bt, f.K, f.sA, f.sB, tm, tn,
-                       a, f.dA, f.dB, f.M, f.N, f.out, f.ldo);
+                       a, f.dA, f.dB, f.M, f.N, f.out, f.ldo, f.fsrc, f.fdst);
     return oz::launch_check(dev, "gemm_crt_kernel");
 }
 

@@ -2,7 +2,7 @@
 // made on the host (the moduli and CRT descriptors of include/oz_hip.h), C = A B through the same
 // stage kernels the C++ backend issues one by one (reference ozaki2.cpp:439-478: scale, slice,
 // products, reconstruction):
-//   flags <- 0; row maxima of A and column maxima of B -> exponent deltas (oz_scale_pair_f64);
+//   row maxima of A and column maxima of B -> exponent deltas and range flags (oz_scale_pair_f64);
 //   residue planes of A and of B^T in OZ_BLOCK tiles (oz2_split_pair_int8);
 //   products reduced to CRT digits in the GEMM epilogue (oz2_gemm_digits);
 //   exact CRT to FP64 (oz2_crt_digits_f64).
@@ -77,16 +77,44 @@ int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, do
     auto* pB = reinterpret_cast<int8_t*>(work + L.planesB);
     auto* dg = work + L.digits;
     const long long sA = (long long)L.Mg * L.Kg, sD = (long long)L.Mg * L.Ng;
-    if (int st = oz_fill_u32(dev, flags, 0u, 2)) return st;
-    // Scheme II rounds the BF16 of the maxima up (reference ozaki2.cpp:143-146)
-    if (int st = oz_scale_pair_f64(dev, A, M, K, lda, B, N, ldb, 1, crt->shift, dA, dB, flags, nullptr)) return st;
-    if (int st = oz2_split_pair_int8(dev, A, M, K, lda, dA, B, N, ldb, dB, mo, pA, pB, L.Mg, L.Ng, L.Kg)) return st;
+    // The scale ORs its flags into two words of the handle that are zero between passes; the last kernel
+    // moves them to the caller's and zeroes them again, so no launch clears anything (a pass that fails on
+    // the way clears them itself).
+    uint32_t* collect = reinterpret_cast<uint32_t*>(dev->queue) + oz_dev::kPassFlags;
+    struct Clear {
+        oz_dev* dev;
+        uint32_t* p;
+        bool armed;
+        ~Clear() {
+            if (armed) {
+                const std::string why = dev->error;
+                (void)oz_fill_u32(dev, p, 0u, 2);
+                dev->error = why;
+            }
+        }
+    } clear{dev, collect, true};
     const long long sB = (long long)L.Ng * L.Kg;
-    if (fused_reconstruction(dev, M, N, L.Kg, crt))
-        return oz::launch_fused(dev, oz::FusedArgs{pA, pB, M, N, L.Kg, sA, sB, crt, dA, dB, C, ldc});
-    if (int st = oz2_gemm_digits(dev, pA, pB, dg, L.Mg, L.Ng, L.Kg, S, L.Ng, sA, sB, sD, crt))
-        return st;
-    return oz2_crt_digits_f64(dev, dg, M, N, L.Ng, sD, crt, dA, dB, C, ldc);
+    const bool fused = fused_reconstruction(dev, M, N, L.Kg, crt);
+    if (prep_takes(dev, mo, M, N, L.Kg)) {
+        // the fused kernel reads rows up to a multiple of 64 only
+        const int Mt = fused ? (M + 63) / 64 * 64 : L.Mg, Nt = fused ? (N + 63) / 64 * 64 : L.Ng;
+        const PrepArgs p{A,  M, K,   lda, Mt, dA, reinterpret_cast<uint8_t*>(pA), sA,         B,
+                         N,  ldb, Nt, dB,  reinterpret_cast<uint8_t*>(pB),         sB, L.Kg, crt->shift, collect};
+        if (int st = launch_prep(dev, p, mo)) return st;
+    } else {
+        // Scheme II rounds the BF16 of the maxima up (reference ozaki2.cpp:143-146)
+        if (int st = oz_scale_pair_f64(dev, A, M, K, lda, B, N, ldb, 1, crt->shift, dA, dB, collect, nullptr)) return st;
+        if (int st = oz2_split_pair_int8(dev, A, M, K, lda, dA, B, N, ldb, dB, mo, pA, pB, L.Mg, L.Ng, L.Kg)) return st;
+    }
+    int st;
+    if (fused) {
+        st = oz::launch_fused(dev, oz::FusedArgs{pA, pB, M, N, L.Kg, sA, sB, crt, dA, dB, C, ldc, collect, flags});
+    } else {
+        st = oz2_gemm_digits(dev, pA, pB, dg, L.Mg, L.Ng, L.Kg, S, L.Ng, sA, sB, sD, crt);
+        if (!st) st = oz::crt_digits_moving_flags(dev, dg, M, N, L.Ng, sD, crt, dA, dB, C, ldc, collect, flags);
+    }
+    clear.armed = st != OZ_OK;
+    return st;
 }
 
 const char* check_args(const double* A, int lda, const double* B, int ldb, const double* C, int ldc, int M, int N,

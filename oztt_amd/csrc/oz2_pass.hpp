@@ -29,4 +29,24 @@ const char* check_args(const double* A, int lda, const double* B, int ldb, const
 int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, double* C, int ldc, int M, int N, int K,
              const oz2_moduli_dev* mo, const oz2_crt_dev* crt, uint32_t* flags, uint8_t* work, const PassLayout& L);
 
+// Deltas and residue planes of both operands in one launch (oz2_prep.hip): A's rows up to Mt and B's
+// columns up to Nt (multiples of 16, zeros past M and N), K padded to Kg; plane strides sA, sB in bytes;
+// flags are ORed into. prep_takes: the rule (short K, a pairwise coprime set).
+struct PrepArgs {
+    const double* A;
+    int M, K, lda, Mt;
+    int32_t* dA;
+    uint8_t* pA;
+    long long sA;
+    const double* B;
+    int N, ldb, Nt;
+    int32_t* dB;
+    uint8_t* pB;
+    long long sB;
+    int Kg, shift;
+    uint32_t* flags;
+};
+bool prep_takes(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int Kg);
+int launch_prep(oz_dev* dev, const PrepArgs& a, const oz2_moduli_dev* mo);
+
 }  // namespace oz2pass

@@ -137,32 +137,32 @@ constexpr int dot_bits() {
 // x = u - q m is in [0, m), and x - (m-1)/2 is the symmetric residue (dinit holds (m-1)/2 plus a
 // multiple of m). Both products are 24-bit multiplies, which run at the full VALU rate. The values
 // returned are x plus a multiple of 2^24 (their low bytes, the ones stored, are x's).
-// The 16 elements of a lane at once, in stages (all dot products, then the quotients, then the
+// The E elements of a lane at once, in stages (all dot products, then the quotients, then the
 // remainders), so that no instruction waits on the one just before it. The first dot product of each
 // element takes dinit from a scalar register (the three-operand form: no copy of dinit per element).
-template <int W>
+template <int W, int E = 16>
 __device__ __forceinline__ void residues_odd_int(const uint32_t (*a)[W], const uint32_t* w, int dinit, uint32_t magic,
                                                  int mneg, int* x) {
     uint32_t wv[W];
 #pragma unroll
     for (int i = 0; i < W; i++) wv[i] = __builtin_amdgcn_readfirstlane(w[i]);
-    int u[16];
+    int u[E];
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
+    for (int e = 0; e < E; e++) {
         asm("v_dot4_i32_i8 %0, %1, %2, %3" : "=v"(u[e]) : "v"(a[e][0]), "v"(wv[0]), "s"(dinit));
 #pragma unroll
         for (int i = 1; i < W; i++) u[e] = __builtin_amdgcn_sdot4((int)a[e][i], (int)wv[i], u[e], false);
     }
     constexpr int sh = 24 - dot_bits<W>();
-    uint32_t q[16];
+    uint32_t q[E];
 #pragma unroll
-    for (int e = 0; e < 16; e++)
+    for (int e = 0; e < E; e++)
         q[e] = (uint32_t)(((unsigned long long)(((uint32_t)u[e] << sh) & 0xFFFFFFu) * (magic & 0xFFFFFFu)) >> 32);
     // u - q m modulo 2^24 as u + q (2^24 - m), one unsigned 24-bit multiply-add (mneg = 2^24 - m;
     // written out, since the compiler widens it to a 32-bit multiply); only the low byte is stored,
     // and it is that of u - q m
 #pragma unroll
-    for (int e = 0; e < 16; e++) asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(x[e]) : "v"(q[e]), "s"(mneg), "v"(u[e]));
+    for (int e = 0; e < E; e++) asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(x[e]) : "v"(q[e]), "s"(mneg), "v"(u[e]));
 }
 
 // The remainder step of residues_odd_int for one sum u in [0, 2^U) (the dot products computed

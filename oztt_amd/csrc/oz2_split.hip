@@ -25,7 +25,7 @@
 // their VALU work (about 12 operations per element and modulus), not by HBM.
 #pragma clang fp contract(off)
 
-#include "oz2_residue.hpp"
+#include "oz2_residue_gen.hpp"
 
 namespace {
 
@@ -99,126 +99,6 @@ __global__ void __launch_bounds__(256) split_tran_kernel(const double* __restric
     }
 }
 
-// Layouts 2/3 (OZ_BLOCK tiles): split_block_kernel of oz_tf32.hpp with this generator: the state of
-// an element is A' in balanced base-256 bytes and its residue modulo the even modulus, if the set
-// has one (from the reference's sequence on the digits); plane s is the residue modulo m_s. The
-// generator runs the planes itself: the even modulus, the odd moduli below 17 (byte dot products and
-// one FP32 reduction, oz2_residue.hpp), then the odd moduli from 17 up four at a time, with their dot
-// products on the matrix cores and the integer remainder step on the VALU.
-//
-// Matrix-core dot products for nd = 3 (8 balanced bytes per element; v_mfma_i32_16x16x64_i8, operand
-// layout as in oz_gemm.hip: lane l holds row l%16 of the first operand and column l%16 of the second,
-// K bytes 16(l/16)..+15 of each; output register r of lane l is row 4(l/16) + r, column l%16). The
-// second operand of lane l is the bytes of two of its own elements, e in its low 8 bytes and e' in its
-// high 8. Row i = 4g + r of the first operand holds, in K chunk g only, the byte weights w_p of modulus
-// p = r%2 of a pair of moduli (symmetric residues of 256^j) over the half h = r/2 of the chunk, and zero
-// elsewhere. So D[4g + r][j] = dinit_p + w_p . (half h of the second operand of lane 16g + j), and
-// output register r of lane l is the dot product of lane l's element (e for r < 2, e' above) with
-// modulus p: every lane gets the four sums of its own two elements and two moduli, 8 MFMAs per pair of
-// moduli for its 16 elements in place of 2 v_dot4 per element and modulus. The sums are exact
-// integers, the same as the v_dot4 chain's. For nd = 4 and 5 (12 and 16 bytes) the v_dot4 chain stays.
-typedef int v4i_t __attribute__((ext_vector_type(4)));
-
-template <int ND>
-struct ResidueGen {
-    static constexpr bool kDrivesPlanes = true;
-    static constexpr int W = balanced_words<ND>();
-    SplitConsts k;
-    struct State {
-        uint32_t a[W];
-        int even;
-    };
-    __device__ __forceinline__ void load(State& st, double x, int32_t d) const {
-        float dig[ND];
-        make_digits<ND>(x, d, dig);
-        balanced_bytes<ND>(dig, st.a);
-        st.even = k.even >= 0 ? residue<ND>(dig, k, k.even) : 0;
-    }
-    // x = r + (m-1)/2 in the low byte: adding 128 - (m-1)/2 keeps every byte in [1, 255] (no carry
-    // into the next one), and xor 0x80 then subtracts 128 from each (two's complement bytes)
-    template <class EMIT>
-    __device__ __forceinline__ void emit_odd(EMIT& emit, int s, const uint32_t* pk) const {
-        const uint32_t badd = k.badd[s];
-        uint32_t w[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) w[c] = (pk[c] + badd) ^ 0x80808080u;
-        emit(s, w);
-    }
-    template <class EMIT>
-    __device__ __forceinline__ void run(State* st, EMIT&& emit) const {
-        uint32_t w[4];
-        if (k.even >= 0) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) w[c] = pack4(st[4 * c].even, st[4 * c + 1].even, st[4 * c + 2].even, st[4 * c + 3].even);
-            emit(k.even, w);
-        }
-        for (int i = 0; i < k.nsmall; i++) {
-            const int s = k.small[i];
-            int v[16];
-#pragma unroll
-            for (int e = 0; e < 16; e++) v[e] = (int)residue_odd<W>(st[e].a, k.w[s], k.m[s], k.rinv[s]);
-#pragma unroll
-            for (int c = 0; c < 4; c++) w[c] = pack4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
-            emit(s, w);
-        }
-        if constexpr (W == 2) {
-            const int lane = threadIdx.x & 63, r = lane & 3;
-            const bool on = (lane >> 4) == ((lane & 15) >> 2);
-            for (int g = 0; g < k.npair; g++) {
-                const int s0 = __builtin_amdgcn_readfirstlane(k.pair[g][0]);
-                const int s1 = __builtin_amdgcn_readfirstlane(k.pair[g][1]);
-                const uint32_t w00 = __builtin_amdgcn_readfirstlane(k.w[s0][0]), w01 = __builtin_amdgcn_readfirstlane(k.w[s0][1]);
-                const uint32_t w10 = __builtin_amdgcn_readfirstlane(k.w[s1][0]), w11 = __builtin_amdgcn_readfirstlane(k.w[s1][1]);
-                const uint32_t lo = (r & 1) ? w10 : w00, hi = (r & 1) ? w11 : w01;
-                const bool h = (r >> 1) != 0;
-                const v4i_t wa = {on && !h ? (int)lo : 0, on && !h ? (int)hi : 0, on && h ? (int)lo : 0, on && h ? (int)hi : 0};
-                const int d0 = k.dinit[s0], d1 = k.dinit[s1];
-                const v4i_t c0 = {d0, d1, d0, d1};
-                const uint32_t mg0 = k.magic[s0], mg1 = k.magic[s1];
-                const int mn0 = k.mneg[s0], mn1 = k.mneg[s1];
-                uint32_t pk0[4], pk1[4];
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    int x0[4], x1[4];
-#pragma unroll
-                    for (int t = 0; t < 2; t++) {
-                        const State& ea = st[4 * c + 2 * t];
-                        const State& eb = st[4 * c + 2 * t + 1];
-                        const v4i_t b = {(int)ea.a[0], (int)ea.a[1], (int)eb.a[0], (int)eb.a[1]};
-                        const v4i_t u = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa, b, c0, 0, 0, 0);
-                        x0[2 * t] = reduce_odd_int<W>(u[0], mg0, mn0);
-                        x1[2 * t] = reduce_odd_int<W>(u[1], mg1, mn1);
-                        x0[2 * t + 1] = reduce_odd_int<W>(u[2], mg0, mn0);
-                        x1[2 * t + 1] = reduce_odd_int<W>(u[3], mg1, mn1);
-                    }
-                    pk0[c] = pack4(x0[0], x0[1], x0[2], x0[3]);
-                    pk1[c] = pack4(x1[0], x1[1], x1[2], x1[3]);
-                }
-                emit_odd(emit, s0, pk0);
-                if (s1 != s0) emit_odd(emit, s1, pk1);
-            }
-        } else {
-            for (int g = 0; g < k.npair; g++)
-#pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    const int s = k.pair[g][p];
-                    if (p == 1 && s == k.pair[g][0]) break;
-                    uint32_t a[16][W];
-#pragma unroll
-                    for (int e = 0; e < 16; e++)
-#pragma unroll
-                        for (int i = 0; i < W; i++) a[e][i] = st[e].a[i];
-                    int v[16];
-                    residues_odd_int<W>(a, k.w[s], k.dinit[s], k.magic[s], k.mneg[s], v);
-                    uint32_t pk[4];
-#pragma unroll
-                    for (int c = 0; c < 4; c++) pk[c] = pack4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
-                    emit_odd(emit, s, pk);
-                }
-        }
-    }
-};
-
 // The reference's sequence for every modulus (sets with more than one even modulus, which a
 // pairwise coprime plan never has): the state is the nd digits.
 template <int ND>
@@ -242,15 +122,6 @@ __global__ void digits_kernel(const double* __restrict__ X, int rows, int cols, 
     make_digits<ND>(X[(size_t)r * ld + c], mode == 0 ? delta[r] : delta[c], dig);
 #pragma unroll
     for (int j = 0; j < ND; j++) out[i * ND + j] = dig[j];
-}
-
-int check_moduli(oz_dev* dev, const oz2_moduli_dev* mo) {
-    if (!mo || mo->S < 1 || mo->S > OZ2_MAXS || mo->nd < 3 || mo->nd > 5)
-        return oz::fail(dev, OZ_ERR_ARG, "oz2_split_int8: invalid moduli descriptor");
-    for (int s = 0; s < mo->S; s++)
-        if (!(mo->m[s] >= 2.0f && mo->m[s] <= 255.0f))
-            return oz::fail(dev, OZ_ERR_ARG, "oz2_split_int8: modulus %g outside the INT8 range", (double)mo->m[s]);
-    return OZ_OK;
 }
 
 template <class GEN>
@@ -292,50 +163,55 @@ int launch_split(oz_dev* dev, const double* X, int rows, int cols, int ld, int m
     return oz::launch_check(dev, "split_tran_kernel");
 }
 
-// Kernel constants of a moduli descriptor (oz2_residue.hpp); *evens counts the even moduli.
-SplitConsts split_consts(const oz2_moduli_dev* mo, int* evens) {
-    SplitConsts k{};
-    k.even = -1;
-    *evens = 0;
-    for (int s = 0; s < mo->S; s++) {
-        k.m[s] = mo->m[s];
-        k.rinv[s] = mo->rinv[s];
-        for (int j = 0; j < 4; j++) k.c[j][s] = mo->c[j][s];
-        // symmetric residues of 256^j modulo m, four to a word (signed bytes)
-        const int m = (int)mo->m[s];
-        if (m % 2 == 1 && m >= 17) {
-            const int U = mo->nd == 3 ? 18 : 19, sh = 24 - U, h = (m - 1) / 2;
-            const long long half = 1ll << (U - 1);
-            k.dinit[s] = (int)((half + m - 1) / m * m + h);
-            k.magic[s] = (uint32_t)(((1ull << (32 - sh)) + m - 1) / m);
-            k.badd[s] = (uint32_t)(128 - h) * 0x01010101u;
-            k.mneg[s] = (1 << 24) - m;
-        }
-        if (m % 2 == 0) {
-            k.even = s;
-            (*evens)++;
-        } else if (m < 17) {
-            k.small[k.nsmall++] = s;
-        } else if (k.npair && k.pair[k.npair - 1][1] < 0) {
-            k.pair[k.npair - 1][1] = s;
-        } else {
-            k.pair[k.npair][0] = s;
-            k.pair[k.npair++][1] = -1;
-        }
-        int p = 1;  // 256^j mod m
-        for (int i = 0; i < 4; i++) {
-            uint32_t word = 0;
-            for (int j = 0; j < 4; j++) {
-                const int sym = p > m / 2 ? p - m : p;
-                word |= (uint32_t)(sym & 0xFF) << (8 * j);
-                p = p * 256 % m;
-            }
-            k.w[s][i] = word;
-        }
+// Both operands in pieces of 64 E elements per wave (the first ceil(nA / 4) workgroups split A): for
+// operands of few blocks, where 16 elements per lane leave SIMDs idle and every wave's chain is long. The
+// whole pass with 16 -> 4 elements per lane, us: 128 x 128 x 512 32.0 -> 27.1, 256 x 256 x 1024 34.0 ->
+// 30.5, 1024^3 (2048 blocks) 58.2 -> 56.6; 2048 x 1024 x 1024 (3072 blocks) 90.2 against 93.7: every wave
+// loads the constants and addresses of its moduli for a quarter of the elements.
+template <int ND, int E>
+__global__ void __launch_bounds__(256) split_pieces_kernel(const double* __restrict__ A, int M, int K, int lda,
+                                                           const int32_t* __restrict__ dA, uint8_t* __restrict__ pA,
+                                                           long long nA, long long sA, const double* __restrict__ B, int N,
+                                                           int ldb, const int32_t* __restrict__ dB,
+                                                           uint8_t* __restrict__ pB, long long nB, long long sB,
+                                                           int kblocks, ResidueGen<ND, E> gen) {
+    constexpr int Q = 16 / E;
+    __shared__ __attribute__((aligned(16))) uint8_t image[4][64 * E];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long gA = (nA + 3) / 4;
+    const bool rows = (long long)blockIdx.x < gA;
+    const long long piece = ((long long)blockIdx.x - (rows ? 0 : gA)) * 4 + wave;
+    if (piece >= (rows ? nA : nB)) return;
+    const int q = (int)(piece % Q), br = (int)(piece / Q / kblocks), kb = (int)(piece / Q % kblocks);
+    double x[E];
+    typename ResidueGen<ND, E>::State st[E];
+    if (rows) {
+        int32_t d[E];
+        load_piece<E, true>(A, M, K, lda, br, kb, q, lane, x);
+#pragma unroll
+        for (int e = 0; e < E; e++) d[e] = dA[min(br * 16 + q * E + e, M - 1)];
+#pragma unroll
+        for (int e = 0; e < E; e++) gen.load(st[e], x[e], d[e]);
+        emit_piece<ND, E, true>(gen, st, pA, sA, br, kblocks, kb, q, lane, image[wave]);
+    } else {
+        load_piece<E, false>(B, K, N, ldb, br, kb, q, lane, x);
+        const int32_t d = dB[min(br * 16 + (lane >> 2), N - 1)];
+#pragma unroll
+        for (int e = 0; e < E; e++) gen.load(st[e], x[e], d);
+        emit_piece<ND, E, false>(gen, st, pB, sB, br, kblocks, kb, q, lane, nullptr);
     }
-    if (k.npair && k.pair[k.npair - 1][1] < 0)  // a last single modulus is paired with itself (stored once)
-        k.pair[k.npair - 1][1] = k.pair[k.npair - 1][0];
-    return k;
+}
+
+template <int ND, int E>
+int launch_pieces(oz_dev* dev, const double* A, int M, int K, int lda, const int32_t* dA, const double* B, int N, int ldb,
+                  const int32_t* dB, const SplitConsts& k, int8_t* pA, int8_t* pB, int Mg, int Ng, int Kg) {
+    const int kblocks = Kg / 64;
+    const long long nA = (long long)(Mg / E) * kblocks, nB = (long long)(Ng / E) * kblocks;
+    hipLaunchKernelGGL((split_pieces_kernel<ND, E>), dim3((unsigned)((nA + 3) / 4 + (nB + 3) / 4)), dim3(256), 0,
+                       dev->stream, A, M, K, lda, dA, reinterpret_cast<uint8_t*>(pA), nA, (long long)Mg * Kg, B, N, ldb, dB,
+                       reinterpret_cast<uint8_t*>(pB), nB, (long long)Ng * Kg, kblocks, ResidueGen<ND, E>{k});
+    return oz::launch_check(dev, "split_pieces_kernel");
 }
 
 template <int ND>
@@ -349,6 +225,9 @@ int launch_pair(oz_dev* dev, const double* A, int M, int K, int lda, const int32
     if (grid > 0x7FFFFFFFll) return oz::fail(dev, OZ_ERR_ARG, "oz2_split_pair_int8: grid too large");
     auto* qA = reinterpret_cast<uint4*>(pA);
     auto* qB = reinterpret_cast<uint4*>(pB);
+    // few blocks: four waves share one (2048 blocks are two waves per SIMD otherwise)
+    if (one_even && nbA + nbB <= 8ll * dev->cus)
+        return launch_pieces<ND, 4>(dev, A, M, K, lda, dA, B, N, ldb, dB, k, pA, pB, Mg, Ng, Kg);
     if (one_even)
         hipLaunchKernelGGL((split_pair_kernel<ResidueGen<ND>>), dim3((unsigned)grid), dim3(256), 0, dev->stream, A, M,
                            K, lda, dA, qA, nbA, sA, B, N, ldb, dB, qB, nbB, sB, kblocks, ResidueGen<ND>{k}, S);

@@ -1,6 +1,7 @@
-"""The whole Scheme II INT8 pass where it computes products and reconstruction in one kernel
-(oz2_gemm_crt.hip: short K, large results), against the same pass run stage by stage through the digits
-(checked against the oracle elsewhere), bit for bit."""
+"""The whole Scheme II INT8 pass where it takes steps together, against the same pass run stage by stage
+(checked against the oracle elsewhere), bit for bit: products and reconstruction in one kernel
+(oz2_gemm_crt.hip: short K, large results), normalization and residues in one (oz2_prep.hip: short K),
+and the range flags that the last kernel hands over."""
 import numpy as np
 import pytest
 
@@ -28,11 +29,45 @@ def operands(M, N, K, seed, phi):
 
 @pytest.mark.parametrize("M,N,K,phi,width", [
     (1500, 1409, 64, 0.5, 0), (2048, 1024, 128, 0.5, 0), (1473, 1472, 250, 1.0, 0), (1440, 1473, 193, 2.0, 0),
-    (700, 3300, 1, 0.5, 0), (1500, 1409, 256, 0.5, 30), (1500, 1409, 256, 4.0, 60),
+    (700, 3300, 1, 0.5, 0), (1500, 1409, 256, 0.5, 30), (1500, 1409, 256, 4.0, 60), (1500, 1409, 256, 0.5, 66),
 ])
 def test_fused_pass_equals_the_stages(dev, M, N, K, phi, width):
     A, B = operands(M, N, K, M + K, phi)
-    p = oz.plan2_int8(A.ravel(), B.ravel(), M, N, K, fixed_bits=width)
+    pass_equals_stages(dev, A, B, M, N, K, width)
+
+
+# deltas and planes in one launch (oz2_prep.hip): 4 elements per lane up to K = 256, 8 up to 512, bands and
+# blocks with padding, 3 to 5 digits
+@pytest.mark.parametrize("M,N,K,width", [
+    (9, 9, 1, 0), (17, 33, 64, 0), (100, 60, 33, 0), (128, 128, 128, 0), (300, 65, 256, 66), (40, 31, 200, 84),
+    (256, 4000, 512, 0), (3900, 300, 449, 0), (2048, 2049, 300, 30),
+])
+def test_prepared_pass_equals_the_stages(dev, M, N, K, width):
+    A, B = operands(M, N, K, M + K, 1.0)
+    pass_equals_stages(dev, A, B, M, N, K, width)
+
+
+def test_range_flags(dev):
+    # the flags of a pass are its own: set by one, clear again in the next; infinities, maxima below 2^-126 and
+    # above the largest BF16 on either side, through every route of the pass
+    for M, N, K in [(64, 48, 100), (64, 48, 700), (1500, 1409, 64), (2048, 2048, 512)]:
+        A, B = operands(M, N, K, 5, 0.5)
+        bad = A.copy()
+        bad[0, 0], bad[5, K - 1], bad[9, 0] = np.inf, 2.0**130, 1.0
+        tiny = B.copy()
+        tiny[:, 1] = 2.0**-200
+        # (A's row 7 and B's column 8 of operands() are below 2^-126 already)
+        clean = A.copy(), B.copy()
+        clean[0][7], clean[1][:, 8] = 1.0, 1.0
+        plan = clean
+        for X, Y, want in [(clean[0], clean[1], (0, 0)), (bad, clean[1], (4 | 1 | 2, 0)), (clean[0], tiny, (0, 2)),
+                           (clean[0], clean[1], (0, 0))]:
+            pass_equals_stages(dev, X, Y, M, N, K, 0, plan, want)
+
+
+def pass_equals_stages(dev, A, B, M, N, K, width, plan=None, want_flags=None):
+    PA, PB = plan or (A, B)
+    p = oz.plan2_int8(PA.ravel(), PB.ravel(), M, N, K, fixed_bits=width)
     moduli = [p.m[i] for i in range(p.S)]
     md, cd = moduli_desc(moduli, p.nd), crt_desc(moduli, p.b, p.nd)
     lda, ldb, ldc = K + 3, N + 5, N + 7
@@ -54,10 +89,14 @@ def test_fused_pass_equals_the_stages(dev, M, N, K, phi, width):
     dev.gemm_digits(pA, pB, dg, Mg, Ng, Kg, p.S, Ng, Mg * Kg, Ng * Kg, Mg * Ng, cd)
     dev.crt_digits(dg, M, N, Ng, Mg * Ng, cd, dA, dB, out, N)
     want = dev.download(out, np.float64, M * N).reshape(M, N)
-    assert not want[1].any() and not want[:, 2].any()
+    if plan is None:
+        assert not want[1].any() and not want[:, 2].any()
     np.testing.assert_array_equal(got[:, :N].view(np.uint64), want.view(np.uint64))
     assert np.all(got[:, N:] == -7.0)
-    np.testing.assert_array_equal(dev.download(fl, np.uint32, 2), dev.download(f2, np.uint32, 2))
+    flags = dev.download(fl, np.uint32, 2)
+    np.testing.assert_array_equal(flags, dev.download(f2, np.uint32, 2))
+    if want_flags:
+        assert tuple(flags) == want_flags
     for x in (bA, bB, bC, fl, work, dA, dB, f2, pA, pB, dg, out):
         x.free()
     dev.bufs.clear()
