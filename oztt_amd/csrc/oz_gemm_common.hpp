@@ -36,24 +36,25 @@ __device__ __forceinline__ void tile_of(int w, int tiles_m, int tiles_n, int nba
 }
 
 // Workgroup -> (batch, tile row, tile column) with every XCD on the same batch at the same time.
-// When the tile count P of a batch is a multiple of 8, batch b's tiles, in the grouped order of
-// tile_of, are cut into 8 contiguous chunks of q = P/8 and XCD x takes chunk x: its j-th workgroup
-// (w = 8j + x) gets tile j % q of its chunk of batch j / q. The XCDs then sweep the batches in
-// step, so the operands in flight are those of one or two batches (at C3 size 2 x 64 MiB of int8
-// planes per batch), which the 256 MB Infinity Cache holds; with tile_of's ranges the 8 XCDs would
-// run 8 different batches and their L2 misses would go to HBM. Within a chunk the ~32 workgroups
-// an XCD runs at a time still cover a compact GROUP_M x 8 block of tiles. Otherwise (P % 8 != 0)
-// this is tile_of. A bijection for any workgroup count of P * nbatch.
+// Workgroups w = b P .. b P + P - 1 run batch b (P tiles), so the XCDs sweep the batches in step and the
+// operands in flight are those of one or two batches (at C3 size 2 x 64 MiB of int8 planes per batch),
+// which the 256 MB Infinity Cache holds; with tile_of's ranges the 8 XCDs would run 8 different batches
+// and their L2 misses would go to HBM. Within a batch each XCD takes one contiguous run of the tiles, in
+// the grouped order of tile_of, so the ~32 workgroups it runs at a time cover a compact GROUP_M x 8
+// block of tiles: XCD x holds the workgroups of the batch with w % 8 == x, q = P/8 of them or q + 1 (the
+// P % 8 XCDs from (b P) % 8 on), and its run starts where those of the XCDs before it end. A bijection for
+// any P and nbatch. (P not a multiple of 8 with tile_of instead: 3520^3 on the FP8 matrix cores, 196
+// tiles per output, 1617 against 1200 us.)
 __device__ __forceinline__ void tile_of_lockstep(int w, int tiles_m, int tiles_n, int nbatch, int& batch, int& tm,
                                                  int& tn) {
     const int P = tiles_m * tiles_n;
-    if (P % XCDS) {
-        tile_of(w, tiles_m, tiles_n, nbatch, batch, tm, tn);
-        return;
-    }
-    const int q = P / XCDS, x = w % XCDS, j = w / XCDS;
-    batch = j / q;
-    const int u = x * q + (j - batch * q);
+    batch = w / P;
+    const int i = w - batch * P, x = w % XCDS;
+    const int q = P / XCDS, r = P % XCDS, s = (w - i) % XCDS;  // s: the XCD of the batch's first workgroup
+    const int k = (x - s) & (XCDS - 1);                        // the XCD's first workgroup of the batch
+    const int wrap = max(s + r - XCDS, 0);                     // XCDs s .. s+r-1 (mod 8) hold one more
+    const int more = min(x, wrap) + min(max(x - s, 0), r - wrap);
+    const int u = x * q + more + (i - k) / XCDS;
     const int group = u / (GROUP_M * tiles_n);
     const int first_m = group * GROUP_M;
     const int gm = min(tiles_m - first_m, GROUP_M);

@@ -23,16 +23,7 @@ __device__ __forceinline__ void small_tile_of(int w, int tiles_m, int tiles_n, i
     if constexpr (MODE != DIAG) {
         tile_of(w, tiles_m, tiles_n, nbatch, batch, tm, tn);
     } else {
-        const int P = tiles_m * tiles_n;
-        batch = w / P;
-        int u = w - batch * P;
-        if (P % XCDS == 0) u = (u % XCDS) * (P / XCDS) + u / XCDS;
-        const int group = u / (GROUP_M * tiles_n);
-        const int first_m = group * GROUP_M;
-        const int gm = min(tiles_m - first_m, GROUP_M);
-        const int v = u % (GROUP_M * tiles_n);
-        tm = first_m + v % gm;
-        tn = v / gm;
+        tile_of_lockstep(w, tiles_m, tiles_n, nbatch, batch, tm, tn);
         batch = nbatch - 1 - batch;
     }
     // wave-uniform, but the divisions run on the VALU
