@@ -66,22 +66,29 @@ void reselect_tail(std::vector<int>& m, double& logM, double need, int m_cap) {
     bool head_even = false;
     for (int x : head) head_even = head_even || (x % 2 == 0);
     const int step = head_even ? 2 : 1;
-    for (int p = 3; p <= m_cap; p += step) {
-        if (!coprime_to_all(p, head)) continue;
-        const double lp = base + std::log2((double)p);
+    // the candidates coprime to the head and their logarithms, once; and a pair's own gcd only when the pair
+    // would be taken (the plan of 64^3: 276 -> 52 us)
+    std::vector<int> cand;
+    std::vector<double> lg;
+    for (int p = 3; p <= m_cap; p += step)
+        if (coprime_to_all(p, head)) {
+            cand.push_back(p);
+            lg.push_back(std::log2((double)p));
+        }
+    for (std::size_t i = 0; i < cand.size(); i++) {
+        const double lp = base + lg[i];
         if (lp >= need && better(1, lp)) {
             best = lp;
-            bp = p;
+            bp = cand[i];
             bq = 0;
             bcost = 1;
         }
-        for (int q = p + step; q <= m_cap; q += step) {
-            if (std::gcd(p, q) != 1 || !coprime_to_all(q, head)) continue;
-            const double lq = lp + std::log2((double)q);
-            if (lq >= need && better(2, lq)) {
+        for (std::size_t j = i + 1; j < cand.size(); j++) {
+            const double lq = lp + lg[j];
+            if (lq >= need && better(2, lq) && std::gcd(cand[i], cand[j]) == 1) {
                 best = lq;
-                bp = p;
-                bq = q;
+                bp = cand[i];
+                bq = cand[j];
                 bcost = 2;
             }
         }
