@@ -69,12 +69,18 @@ __global__ void __launch_bounds__(1024, 8) prep_kernel(const double* __restrict_
     typename ResidueGen<ND, E>::State st[E];
     if (rows) {
 #pragma unroll
-        for (int e = 0; e < E; e++) gen.load(st[e], x[e], delta[q * E + e]);
+        for (int e = 0; e < E; e++) {
+            gen.load(st[e], x[e], delta[q * E + e]);
+            if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
         emit_piece<ND, E, true>(gen, st, pA, sA, br, kblocks, kb, q, lane, image[wave]);
     } else {
         const int d = delta[lane >> 2];
 #pragma unroll
-        for (int e = 0; e < E; e++) gen.load(st[e], x[e], d);
+        for (int e = 0; e < E; e++) {
+            gen.load(st[e], x[e], d);
+            if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
         emit_piece<ND, E, false>(gen, st, pB, sB, br, kblocks, kb, q, lane, nullptr);
     }
 }

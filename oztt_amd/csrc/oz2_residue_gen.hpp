@@ -37,9 +37,20 @@ struct ResidueGen {
     };
     __device__ __forceinline__ void load(State& st, double x, int32_t d) const {
         float dig[ND];
-        make_digits<ND>(x, d, dig);
-        balanced_bytes<ND>(dig, st.a);
-        st.even = k.even >= 0 ? residue<ND>(dig, k, k.even) : 0;
+        if constexpr (ND == 3) {
+            split_integer3(x, d, st.a, dig);
+        } else {
+            make_digits<ND>(x, d, dig);
+            balanced_bytes<ND>(dig, st.a);
+        }
+        // (here and without a branch, held by the empty asm: sunk to its plane, as the compiler would have it, it
+        // keeps every element's digits live that far, 110 registers and more; a set without an even modulus
+        // computes a residue that no plane takes)
+        st.even = residue<ND>(dig, k, max(k.even, 0));
+        if constexpr (ND == 3)
+            asm volatile("" : "+v"(st.even), "+v"(st.a[0]), "+v"(st.a[1]));
+        else
+            asm volatile("" : "+v"(st.even));
     }
     // x = r + (m-1)/2 in the low byte: adding 128 - (m-1)/2 keeps every byte in [1, 255] (no carry
     // into the next one), and xor 0x80 then subtracts 128 from each (two's complement bytes)

@@ -287,7 +287,11 @@ __device__ __forceinline__ void split_block(const double* __restrict__ X, int ro
     }
     typename GEN::State st[16];
 #pragma unroll
-    for (int e = 0; e < 16; e++) gen.load(st[e], xv[e], dv[e]);
+    for (int e = 0; e < 16; e++) {
+        gen.load(st[e], xv[e], dv[e]);
+        if constexpr (drives_planes<GEN>::value)
+            if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four elements' temporaries at a time, not 16
+    }
     if constexpr (drives_planes<GEN>::value) {
         // The planes (17 x 2 x 64 MiB at C3) are read back only by the product kernel, long after
         // the Infinity Cache has turned over: non-temporal stores (2-6% faster split).
