@@ -37,6 +37,7 @@ HIP_SOURCES = {
     "oz_scale.hip": [],
     "oz2_split.hip": ["-fgpu-flush-denormals-to-zero", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "oz2_prep.hip": ["-fgpu-flush-denormals-to-zero", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "oz2_skinny.hip": ["-fgpu-flush-denormals-to-zero", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "oz_gemm.hip": [],
     "oz_gemm_tiles.hip": [],
     "oz2_crt.hip": [],

@@ -285,6 +285,8 @@ __global__ void __launch_bounds__(256) crt_kernel(const int32_t* __restrict__ C,
 // V elements per thread: 4 (one row per blockIdx.y) for large results; 1, with the elements of all rows
 // numbered through, for small ones, which are bound by the latency of one thread's chain (about 200 FP64
 // operations per element) and would leave most lanes idle: 8.8 -> 7.0 us at 256 x 256.
+// TWO (V = 1, at most 16 moduli): a digit is the sum of two, 64 columns apart (the parts of K of
+// oz2_skinny.hip); 2 * 16 * 255 * 2^40 still stays below 2^53.
 // move_flags: thread 0 and 1 of the first workgroup move the range flags of a whole pass (run_pass) from
 // fsrc to fdst and zero fsrc for the next pass.
 __device__ __forceinline__ void move_flags(uint32_t* __restrict__ fsrc, uint32_t* __restrict__ fdst) {
@@ -305,7 +307,7 @@ struct DigitWord<4> {
     using type = uint32_t;
 };
 
-template <int L, int V>
+template <int L, int V, bool TWO = false>
 __global__ void __launch_bounds__(256) crt_digits_kernel(const uint8_t* __restrict__ D, int M, int N, int ldd,
                                                          long long sD, CrtLimbs40 a, const int32_t* __restrict__ dA,
                                                          const int32_t* __restrict__ dB, double* __restrict__ out,
@@ -324,6 +326,10 @@ __global__ void __launch_bounds__(256) crt_digits_kernel(const uint8_t* __restri
     uint32_t v[OZ2_MAXS];
 #pragma unroll
     for (int s = 0; s < OZ2_MAXS; s++) v[s] = d[(long long)min(s, a.S - 1) * sw];
+    if constexpr (TWO) {
+#pragma unroll
+        for (int s = 0; s < OZ2_MAXS; s++) v[s] += d[(long long)min(s, a.S - 1) * sw + 64];
+    }
     double x[V][L];
 #pragma unroll
     for (int e = 0; e < V; e++)
@@ -334,7 +340,7 @@ __global__ void __launch_bounds__(256) crt_digits_kernel(const uint8_t* __restri
         if (s < a.S) {
 #pragma unroll
             for (int e = 0; e < V; e++) {
-                const double k = __hiloint2double(0, (int)((v[s] >> (8 * e)) & 0xFFu));  // k 2^-1074
+                const double k = __hiloint2double(0, (int)(V == 1 ? v[s] : (v[s] >> (8 * e)) & 0xFFu));  // k 2^-1074
 #pragma unroll
                 for (int l = 0; l < L; l++) x[e][l] = __builtin_fma(k, a.Q[s][l], x[e][l]);
             }
@@ -491,7 +497,7 @@ uint64_t limb40(const double* words, int l) {  // bits 40 l .. 40 l + 39 of 8 ex
     }
     return r;
 }
-int crt_limbs40(const CrtLimbs& a, CrtLimbs40& b) {
+int crt_limbs40(const CrtLimbs& a, int parts, CrtLimbs40& b) {
     b = CrtLimbs40{};
     b.S = a.S;
     b.shift = a.shift;
@@ -500,11 +506,11 @@ int crt_limbs40(const CrtLimbs& a, CrtLimbs40& b) {
     for (int l = 0; l < kMaxLimbs40; l++) b.pow40[l] = std::ldexp(1.0, 40 * l);
     b.invM = std::ldexp(a.invM, 90);
     b.delta = a.delta;
-    // bit length of S M (S M < 2^200): the limbs needed
+    // bit length of parts S M (S M < 2^200; at most 16 moduli in two parts): the limbs needed
     uint32_t sm[9] = {};
     uint64_t carry = 0;
     for (int w = 0; w < 8; w++) {
-        const uint64_t p = (uint64_t)(uint32_t)a.Mw[w] * (uint64_t)a.S + carry;
+        const uint64_t p = (uint64_t)(uint32_t)a.Mw[w] * (uint64_t)(a.S * parts) + carry;
         sm[w] = (uint32_t)p;
         carry = p >> 32;
     }
@@ -524,8 +530,12 @@ int crt_limbs40(const CrtLimbs& a, CrtLimbs40& b) {
 
 template <int L>
 int launch_crt_digits(oz_dev* dev, const uint8_t* D, int M, int N, int ldd, long long sD, const CrtLimbs40& a,
-                      const int32_t* dA, const int32_t* dB, double* out, int ldo, uint32_t* fsrc, uint32_t* fdst) {
-    if ((long long)M * N <= 1024ll * dev->cus)  // one element per thread: at most 4 waves per SIMD
+                      const int32_t* dA, const int32_t* dB, double* out, int ldo, uint32_t* fsrc, uint32_t* fdst,
+                      bool two) {
+    if (two)
+        hipLaunchKernelGGL((crt_digits_kernel<L, 1, true>), dim3(oz::ceil_div((long long)M * N, 256)), dim3(256), 0, dev->stream,
+                           D, M, N, ldd, sD, a, dA, dB, out, ldo, fsrc, fdst);
+    else if ((long long)M * N <= 1024ll * dev->cus)  // one element per thread: at most 4 waves per SIMD
         hipLaunchKernelGGL((crt_digits_kernel<L, 1>), dim3(oz::ceil_div((long long)M * N, 256)), dim3(256), 0, dev->stream, D,
                            M, N, ldd, sD, a, dA, dB, out, ldo, fsrc, fdst);
     else
@@ -539,21 +549,21 @@ int launch_crt_digits(oz_dev* dev, const uint8_t* D, int M, int N, int ldd, long
 // launch), so the launch is split in row chunks.
 int crt_launch(oz_dev* dev, const void* C, int kind, int M, int N, int ldc, long long strideC, int nw,
                const CrtLimbs& a, const int32_t* dA, const int32_t* dB, double* out, int ldo, uint32_t* fsrc = nullptr,
-               uint32_t* fdst = nullptr) {
+               uint32_t* fdst = nullptr, bool two = false) {
     const size_t esz = kind == 1 ? 1 : kind == 2 ? 2 : 4;
     if (kind == 1) {
         CrtLimbs40 b;
-        const int L = crt_limbs40(a, b);
+        const int L = crt_limbs40(a, two ? 2 : 1, b);
         for (int i0 = 0; i0 < M; i0 += 65535) {
             const int rows = std::min(65535, M - i0);
             const uint8_t* Di = static_cast<const uint8_t*>(C) + (size_t)i0 * ldc;
             double* oi = out + (long long)i0 * ldo;
             int st;
             switch (L) {
-            case 2: st = launch_crt_digits<2>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst); break;
-            case 3: st = launch_crt_digits<3>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst); break;
-            case 4: st = launch_crt_digits<4>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst); break;
-            default: st = launch_crt_digits<5>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst); break;
+            case 2: st = launch_crt_digits<2>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst, two); break;
+            case 3: st = launch_crt_digits<3>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst, two); break;
+            case 4: st = launch_crt_digits<4>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst, two); break;
+            default: st = launch_crt_digits<5>(dev, Di, rows, N, ldc, strideC, b, dA + i0, dB, oi, ldo, fsrc, fdst, two); break;
             }
             if (st) return st;
             fdst = nullptr;  // moved by the first launch
@@ -580,22 +590,22 @@ int crt_launch(oz_dev* dev, const void* C, int kind, int M, int N, int ldc, long
 
 int crt_f64(oz_dev* dev, const char* name, const void* C, bool digits, int M, int N, int ldc, long long strideC,
             const oz2_crt_dev* crt, const int32_t* dA, const int32_t* dB, double* out, int ldo, uint32_t* fsrc = nullptr,
-            uint32_t* fdst = nullptr) {
+            uint32_t* fdst = nullptr, bool two = false) {
     if (int st = oz::use(dev)) return st;
     if (!C || !crt || !dA || !dB || !out || M <= 0 || N <= 0 || ldc < N || ldo < N || crt->S < 1 ||
         crt->S > OZ2_MAXS || crt->nw < 3 || crt->nw > 8 || (digits && (ldc % 4 || strideC % 4 || ((uintptr_t)C & 3))))
         return oz::fail(dev, OZ_ERR_ARG, "%s: invalid arguments", name);
     CrtLimbs a;
     if (int st = crt_limbs(dev, name, crt, 255u, a)) return st;
-    return crt_launch(dev, C, digits ? 1 : 0, M, N, ldc, strideC, crt->nw, a, dA, dB, out, ldo, fsrc, fdst);
+    return crt_launch(dev, C, digits ? 1 : 0, M, N, ldc, strideC, crt->nw, a, dA, dB, out, ldo, fsrc, fdst, two);
 }
 
 }  // namespace
 
 int oz::crt_digits_moving_flags(oz_dev* dev, const uint8_t* D, int M, int N, int ldd, long long strideD,
                                 const oz2_crt_dev* crt, const int32_t* dA, const int32_t* dB, double* out, int ldo,
-                                uint32_t* fsrc, uint32_t* fdst) {
-    return crt_f64(dev, "oz2_crt_digits_f64", D, true, M, N, ldd, strideD, crt, dA, dB, out, ldo, fsrc, fdst);
+                                uint32_t* fsrc, uint32_t* fdst, bool two) {
+    return crt_f64(dev, "oz2_crt_digits_f64", D, true, M, N, ldd, strideD, crt, dA, dB, out, ldo, fsrc, fdst, two);
 }
 
 extern "C" int oz2_crt_f64(oz_dev* dev, const int32_t* C, int M, int N, int ldc, long long strideC,

@@ -26,9 +26,10 @@ bool fused_limbs(const oz2_crt_dev* crt, int K, int* width, int* limbs);
 int launch_fused(oz_dev* dev, const FusedArgs& f);
 
 // oz2_crt_digits_f64, which also moves the range flags of a whole pass from fsrc to fdst (two device words
-// each) and zeroes fsrc for the next pass, so that no launch has to clear them.
+// each) and zeroes fsrc for the next pass, so that no launch has to clear them. two (at most 16 moduli and
+// 64 columns): the digits are the sums of two, 64 columns apart.
 int crt_digits_moving_flags(oz_dev* dev, const uint8_t* D, int M, int N, int ldd, long long strideD,
                             const oz2_crt_dev* crt, const int32_t* dA, const int32_t* dB, double* out, int ldo,
-                            uint32_t* fsrc, uint32_t* fdst);
+                            uint32_t* fsrc, uint32_t* fdst, bool two = false);
 
 }  // namespace oz

@@ -95,7 +95,12 @@ int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, do
     } clear{dev, collect, true};
     const long long sB = (long long)L.Ng * L.Kg;
     const bool fused = fused_reconstruction(dev, M, N, L.Kg, crt);
-    if (prep_takes(dev, mo, M, N, L.Kg)) {
+    // a matrix on at most 64 columns: B's planes only (64 rows of them)
+    const int parts = skinny_parts(dev, mo, M, N, K);
+    if (parts) {
+        if (int st = oz_scale_pair_f64(dev, A, M, K, lda, B, N, ldb, 1, crt->shift, dA, dB, collect, nullptr)) return st;
+        if (int st = oz2_split_int8(dev, B, K, N, ldb, 1, dB, mo, pB, 3, 64, L.Kg, 64ll * L.Kg)) return st;
+    } else if (prep_takes(dev, mo, M, N, L.Kg)) {
         // the fused kernel reads rows up to a multiple of 64 only
         const int Mt = fused ? (M + 63) / 64 * 64 : L.Mg, Nt = fused ? (N + 63) / 64 * 64 : L.Ng;
         const PrepArgs p{A,  M, K,   lda, Mt, dA, reinterpret_cast<uint8_t*>(pA), sA,         B,
@@ -107,7 +112,11 @@ int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, do
         if (int st = oz2_split_pair_int8(dev, A, M, K, lda, dA, B, N, ldb, dB, mo, pA, pB, L.Mg, L.Ng, L.Kg)) return st;
     }
     int st;
-    if (fused) {
+    if (parts) {
+        st = launch_skinny(dev, A, M, K, lda, dA, pB, L.Kg, dg, L.Ng, sD, parts, mo, crt);
+        if (!st)
+            st = oz::crt_digits_moving_flags(dev, dg, M, N, L.Ng, sD, crt, dA, dB, C, ldc, collect, flags, parts == 2);
+    } else if (fused) {
         st = oz::launch_fused(dev, oz::FusedArgs{pA, pB, M, N, L.Kg, sA, sB, crt, dA, dB, C, ldc, collect, flags});
     } else {
         st = oz2_gemm_digits(dev, pA, pB, dg, L.Mg, L.Ng, L.Kg, S, L.Ng, sA, sB, sD, crt);

@@ -49,4 +49,12 @@ struct PrepArgs {
 bool prep_takes(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int Kg);
 int launch_prep(oz_dev* dev, const PrepArgs& a, const oz2_moduli_dev* mo);
 
+// A matrix on at most 64 columns (oz2_skinny.hip): the digits of A's products with B's residue planes (64 rows
+// of Kg each, OZ_BLOCK tiles) without A's planes. Part p of K (of `parts`, the rule's answer, 0 for a pass it
+// does not take) writes its digits to columns 64 p .. of D's rows; the parts' digits add up. Rows up to a
+// multiple of 64 are written.
+int skinny_parts(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int K);
+int launch_skinny(oz_dev* dev, const double* A, int M, int K, int lda, const int32_t* dA, const int8_t* pB, int Kg,
+                  uint8_t* D, int ldd, long long sD, int parts, const oz2_moduli_dev* mo, const oz2_crt_dev* crt);
+
 }  // namespace oz2pass
