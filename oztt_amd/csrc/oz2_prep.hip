@@ -67,20 +67,29 @@ __global__ void __launch_bounds__(1024, 8) prep_kernel(const double* __restrict_
     }
     __syncthreads();
     typename ResidueGen<ND, E>::State st[E];
+    FarElements far;
     if (rows) {
 #pragma unroll
         for (int e = 0; e < E; e++) {
-            gen.load(st[e], x[e], delta[q * E + e]);
+            gen.load(st[e], x[e], delta[q * E + e], far);
             if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
+        gen.redo(st, far, [&](int e, double& v, int32_t& w) {
+            v = piece_element<E, true>(A, M, K, lda, br, kb, q, e);
+            w = delta[q * E + e];
+        });
         emit_piece<ND, E, true>(gen, st, pA, sA, br, kblocks, kb, q, lane, image[wave]);
     } else {
         const int d = delta[lane >> 2];
 #pragma unroll
         for (int e = 0; e < E; e++) {
-            gen.load(st[e], x[e], d);
+            gen.load(st[e], x[e], d, far);
             if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
+        gen.redo(st, far, [&](int e, double& v, int32_t& w) {
+            v = piece_element<E, false>(B, K, N, ldb, br, kb, q, e);
+            w = d;
+        });
         emit_piece<ND, E, false>(gen, st, pB, sB, br, kblocks, kb, q, lane, nullptr);
     }
 }

@@ -136,7 +136,9 @@ __device__ __forceinline__ void balanced_bytes(const float* dig, uint32_t* a) {
 // The digits are rounded by adding 1.5 2^52 units, ties to even as rint; T holds d0 2^20 + d1 in the low
 // bits of its significand, the multiple of 2^51 in it vanishes modulo 2^64 when shifted up by 20. Values
 // below 2^-41 after scaling have no digits in either form. tests/test_digits_f64.py compares the two.
-__device__ __forceinline__ void split_integer3(double x, int32_t d, uint32_t* a, float* dig) {
+// Holds while d0 leaves T's exponent that of 1.5 2^32, for |x 2^d| < 2^31; the result is T's upper word, by which
+// FarElements tells the others.
+__device__ __forceinline__ uint32_t split_integer3(double x, int32_t d, uint32_t* a, float* dig) {
     const long long u = __double_as_longlong(x);
     const int32_t r = (int32_t)((uint32_t)u << 2) >> 2;
     const double h0 = __builtin_ldexp(__longlong_as_double(u - (long long)r), d);
@@ -156,7 +158,22 @@ __device__ __forceinline__ void split_integer3(double x, int32_t d, uint32_t* a,
     dig[0] = (float)t0;
     dig[1] = (float)t1 * 1048576.0f;
     dig[2] = t2 - 12582912.0f;
+    return (uint32_t)(T >> 32);
 }
+
+// Whether any of some elements was none of split_integer3's: |x 2^d| >= 2^31, an infinity or NaN, or a d from 541 on
+// (there x may be a subnormal, which the procedure takes as zero). The scale leaves elements at most 2^(b - 40)
+// unless a range flag is raised for their row or column, whose planes are still the procedure's.
+struct FarElements {
+    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+    int32_t d = 0;
+    __device__ __forceinline__ void add(uint32_t T, int32_t delta) {
+        lo = min(lo, T);
+        hi = max(hi, T);
+        d = max(d, delta);
+    }
+    __device__ __forceinline__ bool any() const { return lo < 0x41F00000u || hi >= 0x42000000u || d >= 541; }
+};
 
 // |sum_j a_j w_j| < 2^(U-1) for the balanced bytes of A': 2^17 with 8 bytes (nd = 3), 2^18 with up to 16.
 template <int W>

@@ -29,16 +29,19 @@ typedef int v4i_t __attribute__((ext_vector_type(4)));
 template <int ND, int E = 16>
 struct ResidueGen {
     static constexpr bool kDrivesPlanes = true;
+    using Far = FarElements;
     static constexpr int W = balanced_words<ND>();
     SplitConsts k;
     struct State {
         uint32_t a[W];
         int even;
     };
-    __device__ __forceinline__ void load(State& st, double x, int32_t d) const {
+    // PROCEDURE: nd = 3 too through the binary32 digits.
+    template <bool PROCEDURE = ND != 3>
+    __device__ __forceinline__ void load(State& st, double x, int32_t d, Far& far) const {
         float dig[ND];
-        if constexpr (ND == 3) {
-            split_integer3(x, d, st.a, dig);
+        if constexpr (!PROCEDURE) {
+            far.add(split_integer3(x, d, st.a, dig), d);
         } else {
             make_digits<ND>(x, d, dig);
             balanced_bytes<ND>(dig, st.a);
@@ -51,6 +54,23 @@ struct ResidueGen {
             asm volatile("" : "+v"(st.even), "+v"(st.a[0]), "+v"(st.a[1]));
         else
             asm volatile("" : "+v"(st.even));
+    }
+    // After a lane's E elements: where a wave has some that are Far, all go through the procedure, out of line, and are
+    // read again for it by again(e, x, d) (kept for this, the elements would take 20 registers more).
+    template <class AGAIN>
+    __device__ __forceinline__ void redo(State* st, const Far& far, AGAIN again) const {
+        if constexpr (ND == 3)
+            if (__builtin_expect(__ballot(far.any()) != 0, 0)) {
+                Far same;
+#pragma unroll
+                for (int e = 0; e < E; e++) {
+                    double x;
+                    int32_t d;
+                    again(e, x, d);
+                    load<true>(st[e], x, d, same);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
     }
     // x = r + (m-1)/2 in the low byte: adding 128 - (m-1)/2 keeps every byte in [1, 255] (no carry
     // into the next one), and xor 0x80 then subtracts 128 from each (two's complement bytes)
@@ -158,6 +178,18 @@ __device__ __forceinline__ void load_piece(const double* __restrict__ X, int row
         const double v = X[(size_t)min(r0 + e, rows - 1) * ld + cc];
         x[e] = r0 + e < rows && col < cols ? v : 0.0;
     }
+}
+
+// Element e of it, with no address kept since (the lane is taken afresh).
+template <int E, bool ROWS>
+__device__ __forceinline__ double piece_element(const double* __restrict__ X, int rows, int cols, int ld, int br, int kb,
+                                                int q, int e) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int r = (ROWS ? br * 16 + q * E : piece_k0<E>(kb, q, lane)) + e;
+    const int col = ROWS ? kb * 64 + lane : br * 16 + (lane >> 2);
+    const double v = X[(size_t)min(r, rows - 1) * ld + min(col, cols - 1)];
+    return r < rows && col < cols ? v : 0.0;
 }
 
 // E bytes (E / 4 words) to p: a whole block's lane piece non-temporally (as oz_tf32.hpp), shorter ones as

@@ -186,19 +186,28 @@ __global__ void __launch_bounds__(256) split_pieces_kernel(const double* __restr
     const int q = (int)(piece % Q), br = (int)(piece / Q / kblocks), kb = (int)(piece / Q % kblocks);
     double x[E];
     typename ResidueGen<ND, E>::State st[E];
+    FarElements far;
     if (rows) {
         int32_t d[E];
         load_piece<E, true>(A, M, K, lda, br, kb, q, lane, x);
 #pragma unroll
         for (int e = 0; e < E; e++) d[e] = dA[min(br * 16 + q * E + e, M - 1)];
 #pragma unroll
-        for (int e = 0; e < E; e++) gen.load(st[e], x[e], d[e]);
+        for (int e = 0; e < E; e++) gen.load(st[e], x[e], d[e], far);
+        gen.redo(st, far, [&](int e, double& v, int32_t& w) {
+            v = piece_element<E, true>(A, M, K, lda, br, kb, q, e);
+            w = dA[min(br * 16 + q * E + e, M - 1)];
+        });
         emit_piece<ND, E, true>(gen, st, pA, sA, br, kblocks, kb, q, lane, image[wave]);
     } else {
         load_piece<E, false>(B, K, N, ldb, br, kb, q, lane, x);
         const int32_t d = dB[min(br * 16 + (lane >> 2), N - 1)];
 #pragma unroll
-        for (int e = 0; e < E; e++) gen.load(st[e], x[e], d);
+        for (int e = 0; e < E; e++) gen.load(st[e], x[e], d, far);
+        gen.redo(st, far, [&](int e, double& v, int32_t& w) {
+            v = piece_element<E, false>(B, K, N, ldb, br, kb, q, e);
+            w = d;
+        });
         emit_piece<ND, E, false>(gen, st, pB, sB, br, kblocks, kb, q, lane, nullptr);
     }
 }

@@ -253,6 +253,17 @@ struct drives_planes : std::false_type {};
 template <class G>
 struct drives_planes<G, std::void_t<decltype(G::kDrivesPlanes)>> : std::bool_constant<G::kDrivesPlanes> {};
 
+// Generators with a type Far collect in it, as the elements are loaded, whether GEN::redo has to load them again in
+// another way.
+template <class G, class = void>
+struct redoes : std::false_type {
+    struct Far {};
+};
+template <class G>
+struct redoes<G, std::void_t<typename G::Far>> : std::true_type {
+    using Far = typename G::Far;
+};
+
 // Block blk (within a plane, the same for the whole wave) of the operand X; see split_block_kernel.
 template <class GEN, bool TRAN>
 __device__ __forceinline__ void split_block(const double* __restrict__ X, int rows, int cols, int ld, int mode,
@@ -286,12 +297,23 @@ __device__ __forceinline__ void split_block(const double* __restrict__ X, int ro
         }
     }
     typename GEN::State st[16];
+    [[maybe_unused]] typename redoes<GEN>::Far far;
 #pragma unroll
     for (int e = 0; e < 16; e++) {
-        gen.load(st[e], xv[e], dv[e]);
+        if constexpr (redoes<GEN>::value)
+            gen.load(st[e], xv[e], dv[e], far);
+        else
+            gen.load(st[e], xv[e], dv[e]);
         if constexpr (drives_planes<GEN>::value)
             if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four elements' temporaries at a time, not 16
     }
+    if constexpr (redoes<GEN>::value)
+        gen.redo(st, far, [&](int e, double& x, int32_t& d) {  // as the edge blocks' loads above
+            const int xr = min(xr0 + e, rows - 1), xc = min(xc0, cols - 1);
+            const double v = X[(size_t)xr * ld + xc];
+            x = xr0 + e < rows && xc0 < cols ? v : 0.0;
+            d = mode == 0 ? delta[xr] : delta[xc];
+        });
     if constexpr (drives_planes<GEN>::value) {
         // The planes (17 x 2 x 64 MiB at C3) are read back only by the product kernel, long after
         // the Infinity Cache has turned over: non-temporal stores (2-6% faster split).

@@ -44,7 +44,11 @@ def reference(x, d):
 
 
 def split_integer3(x, d):
-    """The kernel's sequence."""
+    return integer_and_sum(x, d)[0]
+
+
+def integer_and_sum(x, d):
+    """The kernel's sequence: A', and T, whose upper word says whether the sequence holds."""
     u = x.view(np.int64)
     r = ((u & 0xFFFFFFFF) << 34) >> 34  # bits 0..29, signed
     h0 = np.ldexp((u - r).view(np.float64), d)
@@ -60,7 +64,7 @@ def split_integer3(x, d):
     f = (hi2 + mid).astype(F)
     fb = (f.astype(np.float64) * 2.0**40 + 12582912.0).astype(F).view(np.int32).astype(np.int64)  # one rounding: exact below 2^53
     T = T1 + t0
-    return ((T.view(np.uint64) << np.uint64(20)).view(np.int64)) + (fb - 0x4B400000)
+    return ((T.view(np.uint64) << np.uint64(20)).view(np.int64)) + (fb - 0x4B400000), T
 
 
 def check(x, d):
@@ -106,3 +110,32 @@ def test_zero_and_extremes():
     x = np.array([0.0, -0.0, 5e-324, -2.0**-1022, 2.0**-1060, 1.0, -1.0, 2.0**-41, 2.0**-40, -2.0**-20])
     for d in (0, 16, 20, 142):
         check(x[:5] if d > 20 else x, np.int64(d))
+
+
+def test_far_elements_are_told_apart():
+    """Every element that Far passes has the procedure's A', whatever its size and delta, and no element below 2^30
+    (what the scale leaves, unless a range flag is raised) is sent through the procedure."""
+    rng = np.random.default_rng(3)
+    n = 400000
+    for spread in (40, 120, 2000):
+        x = rng.integers(0, 2**64, n, dtype=np.uint64).view(np.float64).copy()  # infinities and NaN among them
+        u = x.view(np.uint64)
+        near_range = rng.random(n) < 0.8
+        E = np.clip(1023 + rng.integers(-spread, spread + 1, n), 0, 2047).astype(np.uint64)
+        u[near_range] = (u[near_range] & np.uint64((1 << 63) | ((1 << 52) - 1))) | (E[near_range] << np.uint64(52))
+        x[:16] = [np.inf, -np.inf, np.nan, -np.nan, 0.0, -0.0, 5e-324, 1.7976931348623157e308, 2.0**31, -(2.0**31), 2.0**30,
+                  2.0**32, -(2.0**32), 1.5 * 2.0**32, -1.5 * 2.0**32, -(2.0**33)]
+        d = rng.integers(-60, 60, n)
+        some = rng.random(n) < 0.1
+        d[some] = rng.integers(-1100, 1100, int(some.sum()))
+        d[:16] = 0
+        with np.errstate(all="ignore"):
+            got, T = integer_and_sum(x, d)
+            want = reference(x, d)
+            size = np.abs(np.ldexp(x, d))
+        hi = T.view(np.uint64) >> np.uint64(32)
+        passed = (hi >= 0x41F00000) & (hi < 0x42000000) & (d < 541)
+        assert 0.01 < passed.mean() < 0.99
+        bad = np.flatnonzero(passed & (got != want))
+        assert not bad.size, (x[bad[:3]], d[bad[:3]])
+        assert passed[(size < 2.0**30) & (d < 541)].all()
