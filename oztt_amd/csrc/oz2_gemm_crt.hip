@@ -331,8 +331,10 @@ void constants(const oz2_crt_dev* crt, int w, FusedCrt<L>& a) {
     }
 }
 
-// M = prod m_s and Q_s m_s = M for every modulus (the descriptor is the caller's).
+// M = prod m_s, Q_s m_s = M for every modulus, and S M within the nw words of the accumulator (the descriptor is the
+// caller's: what is not so goes to the general route, where oz2_crt_digits_f64 refuses it).
 bool consistent(const oz2_crt_dev* crt) {
+    if (crt->nw < 3 || crt->nw > 8) return false;
     uint32_t M[9] = {1};
     for (int s = 0; s < crt->S; s++) {
         uint64_t carry = 0;
@@ -345,6 +347,13 @@ bool consistent(const oz2_crt_dev* crt) {
     for (int k = 0; k < 8; k++)
         if (M[k] != crt->Mw[k]) return false;
     if (M[8]) return false;
+    uint64_t over = 0;
+    for (int k = 0; k < 8; k++) {
+        const uint64_t p = (uint64_t)M[k] * (uint64_t)crt->S + over;
+        if (k >= crt->nw && (uint32_t)p) return false;
+        over = p >> 32;
+    }
+    if (over) return false;
     for (int s = 0; s < crt->S; s++) {
         uint64_t carry = 0;
         for (int k = 0; k < 8; k++) {
