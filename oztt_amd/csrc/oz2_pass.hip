@@ -20,6 +20,13 @@
 namespace oz2pass {
 
 namespace {
+__global__ void move_flags_kernel(uint32_t* __restrict__ from, uint32_t* __restrict__ to) {
+    if (threadIdx.x < 2) {
+        to[threadIdx.x] = from[threadIdx.x];
+        from[threadIdx.x] = 0u;
+    }
+}
+
 size_t round256(size_t v) { return (v + 255) / 256 * 256; }
 }  // namespace
 
@@ -78,21 +85,19 @@ int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, do
     auto* dg = work + L.digits;
     const long long sA = (long long)L.Mg * L.Kg, sD = (long long)L.Mg * L.Ng;
     // The scale ORs its flags into two words of the handle that are zero between passes; the last kernel
-    // moves them to the caller's and zeroes them again, so no launch clears anything (a pass that fails on
-    // the way clears them itself).
+    // moves them to the caller's and zeroes them again, so no launch clears anything. A pass that fails on the
+    // way moves them itself: the caller's words are what the scale found, zero if it did not run.
     uint32_t* collect = reinterpret_cast<uint32_t*>(dev->queue) + oz_dev::kPassFlags;
-    struct Clear {
+    struct HandOver {
         oz_dev* dev;
-        uint32_t* p;
+        uint32_t *from, *to;
         bool armed;
-        ~Clear() {
-            if (armed) {
-                const std::string why = dev->error;
-                (void)oz_fill_u32(dev, p, 0u, 2);
-                dev->error = why;
-            }
+        ~HandOver() {
+            if (!armed) return;
+            hipLaunchKernelGGL(move_flags_kernel, dim3(1), dim3(64), 0, dev->stream, from, to);
+            (void)hipGetLastError();  // (the pass reports why it failed)
         }
-    } clear{dev, collect, true};
+    } failed{dev, collect, flags, true};
     const long long sB = (long long)L.Ng * L.Kg;
     const bool fused = fused_reconstruction(dev, M, N, L.Kg, crt);
     // a matrix on at most 64 columns: B's planes only (64 rows of them)
@@ -122,7 +127,7 @@ int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, do
         st = oz2_gemm_digits(dev, pA, pB, dg, L.Mg, L.Ng, L.Kg, S, L.Ng, sA, sB, sD, crt);
         if (!st) st = oz::crt_digits_moving_flags(dev, dg, M, N, L.Ng, sD, crt, dA, dB, C, ldc, collect, flags);
     }
-    clear.armed = st != OZ_OK;
+    failed.armed = st != OZ_OK;
     return st;
 }
 

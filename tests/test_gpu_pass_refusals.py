@@ -47,9 +47,13 @@ def test_accumulator_words(dev, M, N, K, nw):
     # 15 moduli: S M takes 122 bits, four words
     p = Pass(dev, M, N, K)
     p.cd.nw = nw
-    refused, C, _ = p.run()
+    refused, C, flags = p.run()
     assert refused and "oz2_crt_digits_f64" in refused
     assert np.all(C == 3.0)
+    assert flags == (4, 1)  # the refusal comes after the scale: what it found, as in a pass that runs
+    p.cd.nw = 4
+    p.A[3, 0] = p.B[1, 2] = 1.0
+    assert p.run()[2] == (0, 0)  # and the next pass finds nothing of it
 
 
 @pytest.mark.parametrize("M,N,K", ROUTES)
