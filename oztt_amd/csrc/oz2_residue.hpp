@@ -55,22 +55,26 @@ __device__ __forceinline__ float mod_round(float v, float m, float rinv) {
     return __builtin_fmaf(-q, m, v);  // exact: q*m and v - q*m are integers below 2^24
 }
 
-// Step 3 for one modulus: the symmetric residue (|r| <= floor(m/2) + 1) as an FP32 integer.
+// Step 3 for one modulus m (ri: its reciprocal, c: 2^(20 (j + 1)) mod m): the symmetric residue (|r| <= floor(m/2) + 1)
+// as an FP32 integer.
 template <int ND>
-__device__ __forceinline__ float residue_f(const float* dig, const SplitConsts& k, int s) {
-    const float m = k.m[s], ri = k.rinv[s];
+__device__ __forceinline__ float residue_f(const float* dig, float m, float ri, float c0, float c1, float c2, float c3) {
     float acc = dig[ND - 1];
-    acc = __builtin_fmaf(mod_round(dig[ND - 2], m, ri), k.c[0][s], acc);
-    acc = __builtin_fmaf(mod_round(dig[ND - 3], m, ri), k.c[1][s], acc);
+    acc = __builtin_fmaf(mod_round(dig[ND - 2], m, ri), c0, acc);
+    acc = __builtin_fmaf(mod_round(dig[ND - 3], m, ri), c1, acc);
     if (ND >= 4) {
         acc = mod_round(acc, m, ri);
         if (ND >= 5) {
-            acc = __builtin_fmaf(mod_round(dig[0], m, ri), k.c[3][s], acc);
+            acc = __builtin_fmaf(mod_round(dig[0], m, ri), c3, acc);
             acc = mod_round(acc, m, ri);
         }
-        acc = __builtin_fmaf(mod_round(dig[ND - 4], m, ri), k.c[2][s], acc);
+        acc = __builtin_fmaf(mod_round(dig[ND - 4], m, ri), c2, acc);
     }
     return mod_round(acc, m, ri);
+}
+template <int ND>
+__device__ __forceinline__ float residue_f(const float* dig, const SplitConsts& k, int s) {
+    return residue_f<ND>(dig, k.m[s], k.rinv[s], k.c[0][s], k.c[1][s], k.c[2][s], k.c[3][s]);
 }
 template <int ND>
 __device__ __forceinline__ int residue(const float* dig, const SplitConsts& k, int s) {
@@ -165,14 +169,13 @@ __device__ __forceinline__ uint32_t split_integer3(double x, int32_t d, uint32_t
 // (there x may be a subnormal, which the procedure takes as zero). The scale leaves elements at most 2^(b - 40)
 // unless a range flag is raised for their row or column, whose planes are still the procedure's.
 struct FarElements {
-    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+    uint32_t top = 0;
     int32_t d = 0;
     __device__ __forceinline__ void add(uint32_t T, int32_t delta) {
-        lo = min(lo, T);
-        hi = max(hi, T);
+        top = max(top, T - 0x41F00000u);
         d = max(d, delta);
     }
-    __device__ __forceinline__ bool any() const { return lo < 0x41F00000u || hi >= 0x42000000u || d >= 541; }
+    __device__ __forceinline__ bool any() const { return top >= 0x100000u || d >= 541; }
 };
 
 // |sum_j a_j w_j| < 2^(U-1) for the balanced bytes of A': 2^17 with 8 bytes (nd = 3), 2^18 with up to 16.

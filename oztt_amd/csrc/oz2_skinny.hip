@@ -14,7 +14,9 @@
 //     lane, two waves per SIMD: with all moduli in one wave, one per SIMD, every latency showed, 1.9x slower);
 //   - B's blocks (4 S KB per K block, 64 rows of planes) come into LDS once for the 8 waves, a block ahead.
 // A's residues may be any representatives (the products are reduced), so the even modulus goes the way of the
-// odd ones, whatever the planes' sequence makes of a tie, and a small modulus that of a multiple.
+// odd ones, whatever the planes' sequence makes of a tie, and a small modulus that of a multiple. A workgroup that met
+// an element without a place in the digits (its row has a range flag) computes its rows once more from the planes' own
+// residues, so that flagged rows come out as the stages give them too.
 // Bound by the VALU work of the residues (54% busy) and, for A's 64 KB rows, by the memory channels: without the
 // reads of A the pass takes 88 us less, without B's copies 46, without the residues' VALU work 29.
 // Whole pass, us, with planes -> here: 8192 x 64 x 8192: 645 -> 405; 8192 x 1 x 8192: 632 -> 413; 12288 x 64 x
@@ -43,6 +45,8 @@ constexpr int kBuf = kMaxS * 4096;             // a K block of B's planes
 struct SkinnyConsts {
     uint32_t w[kMaxS][2], magic[kMaxS];
     int init[kMaxS], mneg[kMaxS];
+    int even;  // the even modulus of the set or -1, with the constants of its sequence on the digits (residue_f)
+    float m, rinv, c0, c1;
 };
 
 __device__ __forceinline__ int residue_byte(int u, int v, uint32_t magic, int mneg) {
@@ -113,13 +117,14 @@ __global__ void __launch_bounds__(512) skinny_kernel(const double* __restrict__ 
             }
         }
     };
+    FarElements far;  // over all elements of this thread
     auto convert = [&](const double* x, v4i* g) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             uint32_t a0[2], a1[2];
             float dig[3];
-            split_integer3(live ? x[2 * j] : 0.0, delta, a0, dig);
-            split_integer3(live ? x[2 * j + 1] : 0.0, delta, a1, dig);
+            far.add(split_integer3(live ? x[2 * j] : 0.0, delta, a0, dig), 0);
+            far.add(split_integer3(live ? x[2 * j + 1] : 0.0, delta, a1, dig), 0);
             g[j] = v4i{(int)a0[0], (int)a0[1], (int)a1[0], (int)a1[1]};
         }
     };
@@ -203,6 +208,51 @@ __global__ void __launch_bounds__(512) skinny_kernel(const double* __restrict__ 
     }
     wait_vmcnt_lgkm0<0>();  // the last block's copies, issued twice
     __syncthreads();
+    // Elements that are Far (an operand with a range flag) are what the procedure makes of them, also in the even
+    // modulus, whose sequence on the digits then is no residue of A': rows with such elements once more, their residues
+    // by the functions of the planes and through LDS.
+    int* seen = reinterpret_cast<int*>(states);
+    if (lane == 0) seen[wave] = 0;
+    if (far.any() || delta >= 541) seen[wave] = 1;
+    __syncthreads();
+    bool again = false;
+#pragma unroll
+    for (int i = 0; i < 8; i++) again |= seen[i] != 0;
+    if (__builtin_expect(again, 0)) {
+#pragma unroll
+        for (int i = 0; i < 2 * P; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = v4i{0, 0, 0, 0};
+        for (int i = 0; i < steps; i++) {
+            load(x, st0 + i);
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                uint32_t a[2];
+                float dig[3];
+                make_digits<3>(live ? x[e] : 0.0, delta, dig);
+                balanced_bytes<3>(dig, a);
+                int8_t* at = lds + 64 * lrow + 2 * lq + 16 * (e >> 1) + (e & 1);
+                for (int s = 0; s < S; s++) {
+                    const float m = (float)((1 << 24) - k.mneg[s]);
+                    at[4096 * s] = (int8_t)(int)(s == k.even ? residue_f<3>(dig, k.m, k.rinv, k.c0, k.c1, 0.0f, 0.0f)
+                                                             : residue_odd<2>(a, k.w[s], m, 1.0f / m));
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int g = 0; g < 2 * P; g++) {
+                const int s = min(s0 + g, S - 1);
+                const v4i f = *reinterpret_cast<const v4i*>(lds + 4096 * s + 64 * (16 * band + r) + 16 * c);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    acc[g][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                        f, *reinterpret_cast<const v4i*>(pB + ((long long)s * sB + ((long long)j * nk + st0 + i) * 1024 + foff)),
+                        acc[g][j], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
     // digits through 4 KB of the ring per wave (its LDS operations are in order), 16 sums per lane and modulus
     int32_t* tile = reinterpret_cast<int32_t*>(lds) + wave * 1024;
 #pragma unroll
@@ -231,7 +281,9 @@ namespace oz2pass {
 // from where normalization and residues are no longer one launch (K > 512, oz2_prep.hip) and its workgroups, one
 // per CU, fill the chip: with 192 of them (M = 6144, two parts) the pass takes 77 us against 95 at K = 1024.
 int skinny_parts(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int K) {
-    if (N > 64 || mo->nd != 3 || mo->S > kMaxS || K < 1024) return 0;
+    int evens = 0;  // (more than one, and the planes are all of the sequence on the digits)
+    for (int s = 0; s < mo->S; s++) evens += (int)mo->m[s] % 2 == 0;
+    if (N > 64 || mo->nd != 3 || mo->S > kMaxS || K < 1024 || evens > 1) return 0;
     const long long groups = (M + 63ll) / 64, cus = dev->cus;
     for (int parts = 1; parts <= 2; parts++) {
         const long long w = groups * parts, rounds = (w + cus - 1) / cus;
@@ -243,6 +295,15 @@ int skinny_parts(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int 
 int launch_skinny(oz_dev* dev, const double* A, int M, int K, int lda, const int32_t* dA, const int8_t* pB, int Kg,
                   uint8_t* D, int ldd, long long sD, int parts, const oz2_moduli_dev* mo, const oz2_crt_dev* crt) {
     SkinnyConsts k{};
+    k.even = -1;
+    for (int s = 0; s < mo->S; s++)
+        if ((int)mo->m[s] % 2 == 0) {
+            k.even = s;
+            k.m = mo->m[s];
+            k.rinv = mo->rinv[s];
+            k.c0 = mo->c[0][s];
+            k.c1 = mo->c[1][s];
+        }
     for (int i = 0; i < kMaxS; i++) {
         const int m1 = (int)mo->m[std::min(i, mo->S - 1)], m = 255 / m1 * m1, h = m / 2;
         int p = 1;  // 256^j mod m, symmetric

@@ -76,12 +76,38 @@ def test_range_flags(dev):
             pass_equals_stages(dev, X, Y, M, N, K, 0, plan, want)
 
 
-def pass_equals_stages(dev, A, B, M, N, K, width, plan=None, want_flags=None):
-    # (the row of an infinity has no result: its elements are whatever the residues of no integer give)
-    rows = np.isfinite(A).all(axis=1) if N <= 64 and K >= 1024 else np.ones(M, bool)
+# Rows and columns with a range flag: infinities, NaN, values above the largest BF16, alone and beside values whose
+# scaled digits do not fit (the even modulus of such elements is no residue of their A'). One size of every route; of
+# the narrow one both parts of K, few moduli, and 2 as the even one.
+@pytest.mark.parametrize("M,N,K,width,moduli", [
+    (100, 90, 120, 0, None), (300, 4000, 512, 0, None), (300, 300, 700, 0, None), (1500, 1409, 64, 0, None),
+    (6100, 20, 1030, 0, None), (12290, 64, 1100, 0, None), (6081, 64, 1999, 0, None), (6100, 33, 1024, 30, None),
+    (6144, 17, 1100, 0, [255, 253, 251, 247, 2, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193]),
+    (6144, 9, 1100, 0, [255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193]),
+])
+def test_flagged_operands_equal_the_stages(dev, M, N, K, width, moduli):
+    A, B = operands(M, N, K, M + K, 0.5)
+    rng = np.random.default_rng(K)
+    for X, n, axis in ((A, K, 0), (B.T, K, 1)):
+        X[0, n - 1], X[3, n // 2] = np.inf, np.nan
+        if len(X) < 16:
+            continue
+        X[9, 0] = 2.0 ** 130
+        X[10] *= 2.0 ** 140
+        X[11] *= np.exp2(rng.integers(0, 60, n))
+        X[11, 0] = -np.inf
+        X[12] *= np.exp2(rng.integers(-60, 1000, n))
+        X[13] = 2.0 ** -1060
+        X[15, n - 1] = 2.0 ** 128
+    A[M - 1, K - 1] = np.nan
+    pass_equals_stages(dev, A, B, M, N, K, width, operands(M, N, K, 1, 0.5), moduli=moduli)
+
+
+def pass_equals_stages(dev, A, B, M, N, K, width, plan=None, want_flags=None, moduli=None):
     PA, PB = plan or (A, B)
     p = oz.plan2_int8(PA.ravel(), PB.ravel(), M, N, K, fixed_bits=width)
-    moduli = [p.m[i] for i in range(p.S)]
+    moduli = moduli or [p.m[i] for i in range(p.S)]
+    S = len(moduli)
     md, cd = moduli_desc(moduli, p.nd), crt_desc(moduli, p.b, p.nd)
     lda, ldb, ldc = K + 3, N + 5, N + 7
     a, b = np.zeros((M, lda)), np.zeros((K, ldb))
@@ -89,22 +115,22 @@ def pass_equals_stages(dev, A, B, M, N, K, width, plan=None, want_flags=None):
     bA, bB = dev.upload(a), dev.upload(b)
     bC = dev.upload(np.full((M, ldc), -7.0))
     fl = dev.alloc(16)
-    need = dev.gemm_f64_workspace(M, N, K, p.S)
+    need = dev.gemm_f64_workspace(M, N, K, S)
     work = dev.alloc(need)
     dev.gemm_f64(bA, lda, bB, ldb, bC, ldc, M, N, K, md, cd, fl, work, need)
     got = dev.download(bC, np.float64, M * ldc).reshape(M, ldc)
     # the stages
     Mg, Ng, Kg = -(-M // 256) * 256, -(-N // 256) * 256, -(-K // 64) * 64
     dA, dB, f2 = dev.alloc(4 * M), dev.alloc(4 * N), dev.upload(np.zeros(2, np.uint32))
-    pA, pB, dg, out = dev.alloc(p.S * Mg * Kg), dev.alloc(p.S * Ng * Kg), dev.alloc(p.S * Mg * Ng), dev.alloc(8 * M * N)
+    pA, pB, dg, out = dev.alloc(S * Mg * Kg), dev.alloc(S * Ng * Kg), dev.alloc(S * Mg * Ng), dev.alloc(8 * M * N)
     dev.scale_pair(bA, M, K, lda, bB, N, ldb, 1, cd.shift, dA, dB, f2)
     dev.split_pair_int8(bA, M, K, lda, dA, bB, N, ldb, dB, md, pA, pB, Mg, Ng, Kg)
-    dev.gemm_digits(pA, pB, dg, Mg, Ng, Kg, p.S, Ng, Mg * Kg, Ng * Kg, Mg * Ng, cd)
+    dev.gemm_digits(pA, pB, dg, Mg, Ng, Kg, S, Ng, Mg * Kg, Ng * Kg, Mg * Ng, cd)
     dev.crt_digits(dg, M, N, Ng, Mg * Ng, cd, dA, dB, out, N)
     want = dev.download(out, np.float64, M * N).reshape(M, N)
     if plan is None:
         assert not want[1].any() and not want[:, 2].any()
-    np.testing.assert_array_equal(got[rows, :N].view(np.uint64), want[rows].view(np.uint64))
+    np.testing.assert_array_equal(got[:, :N].view(np.uint64), want.view(np.uint64))
     assert np.all(got[:, N:] == -7.0)
     flags = dev.download(fl, np.uint32, 2)
     np.testing.assert_array_equal(flags, dev.download(f2, np.uint32, 2))
