@@ -48,6 +48,7 @@ HIP_SOURCES = {
     "oz2_gemm_f8.hip": [],
     "oz2_pass.hip": [],
     "oz2_noalloc.hip": [],
+    "oz_rules.hip": [],
 }
 HOST_FLAGS = ["-std=c++20", "-O2", "-fPIC", "-ffp-contract=off", "-fno-fast-math", "-fopenmp",
               "-Wall", "-Wextra", f"-I{INCLUDE}", f"-I{CSRC / 'host'}"]

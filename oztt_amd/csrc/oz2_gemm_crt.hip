@@ -13,7 +13,7 @@
 //     V = sum_s C_s W_s,   W_s = y_s Q_s < M  (so V == C' modulo M),
 // in L limbs of w bits held as exact doubles, w such that S max|C_s| 2^w <= 2^52: one conversion and L
 // FMAs per element and modulus, in place of a digit (four FP64 operations, packing, LDS, a store), a load
-// and its L accumulations. t = rint(V / M) is now up to S max|C_s| and its estimate good to 2^-22 (the
+// and its L accumulations. t = rint(V / M) is now up to S max|C_s| and its estimate good to 2^-20.6 (w >= 24; the
 // threshold of the exact comparison, delta, is 2^-20); the rest of the finish is that of oz2_crt.hip.
 //
 // It is bound by the FP64 pipe (L + 1 operations per element and modulus, about 110 for the finish) while
@@ -380,13 +380,15 @@ int launch(oz_dev* dev, const oz::FusedArgs& f, int w) {
 
 namespace oz {
 
-// Limb width and count: S max|C_s| 2^w <= 2^52 with |C_s| <= K 127^2, and L w bits for M.
+// Limb width and count: S max|C_s| 2^w <= 2^52 with |C_s| <= K 127^2, and L w bits for M. w >= 24, so that the
+// quotient V / M < 2^28 is good to 2^-20.6 (at most 2 L + 8 roundings on the way, each within 2^-53 of 2^28) and
+// finish settles every neighbour that delta, 2^-20, leaves open: with w = 18 (10 moduli, K = 65536) it is off by more.
 bool fused_limbs(const oz2_crt_dev* crt, int K, int* width, int* limbs) {
     const int w = 52 - bit_length((uint64_t)crt->S * K * 127 * 127);
     int bits = 0;
     for (int k = 7; k >= 0 && !bits; k--)
         if (crt->Mw[k]) bits = 32 * k + 32 - __builtin_clz(crt->Mw[k]);
-    if (w < 16 || !bits) return false;
+    if (w < 24 || !bits) return false;
     const int L = std::max(4, (bits + w - 1) / w);
     *width = w;
     *limbs = L;
