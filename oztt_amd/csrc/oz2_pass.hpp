@@ -53,6 +53,12 @@ int launch_prep(oz_dev* dev, const PrepArgs& a, const oz2_moduli_dev* mo);
 // of Kg each, OZ_BLOCK tiles) without A's planes. Part p of K (of `parts`, the rule's answer, 0 for a pass it
 // does not take) writes its digits to columns 64 p .. of D's rows; the parts' digits add up. Rows up to a
 // multiple of 64 are written.
+// The constants of modulus m1 in that kernel (oz2_skinny.hip, SkinnyConsts).
+struct NarrowModulus {
+    uint32_t w[2], magic;
+    int init, mneg;
+};
+NarrowModulus narrow_modulus(int m1);
 int skinny_parts(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int K);
 int launch_skinny(oz_dev* dev, const double* A, int M, int K, int lda, const int32_t* dA, const int8_t* pB, int Kg,
                   uint8_t* D, int ldd, long long sD, int parts, const oz2_moduli_dev* mo, const oz2_crt_dev* crt);

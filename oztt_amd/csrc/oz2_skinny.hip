@@ -33,15 +33,16 @@ using namespace ozg;
 constexpr int kMaxS = 16;
 constexpr int kBuf = kMaxS * 4096;             // a K block of B's planes
 
-// Constants of a modulus m (129 <= m <= 255, h = m / 2; for a smaller modulus of the set, m is its largest multiple
+// Constants of a modulus m (128 <= m <= 255, h = m / 2; for a smaller modulus of the set, m is its largest multiple
 // up to 255: the residues are representatives). With u = dot + 2 h + 2 L m (one MFMA) and
 // v = u + dot = 2 (dot + h + L m) (a second one on top), q = floor(v magic / 2^32), magic = ceil(2^31 / m) < 2^24,
-// is floor((dot + h) / m) + L exactly (v < 2^20, so the excess of magic adds less than 2^-12 < 1 / m; checked for
-// every m and every dot), and
+// is floor((dot + h) / m) + L exactly (v < 2^20, so the excess of magic adds less than 2^-12 < 1 / m), and
 // u - q m = r + (2 h + L m) with r = dot + h mod m - h the symmetric residue. L m >= 2^17 > |dot| is chosen with
 // 2 h + L m = 0 mod 256: the low byte of u - q m is r. So a residue takes two VALU instructions (24-bit multiply
 // high and multiply-add) and its share of the packing, 2.75 against the 4.25 of reduce_odd_int with its shift
 // and its offset, and the matrix cores, idle otherwise, make v. Both parities of m: for even m, h + h = m.
+// m = 128 has no such magic (2^24): with 0, q = 0 and the byte is u's own, congruent to dot modulo 128 since 256 is a
+// multiple of it, at most 128 in magnitude beside B's 64. tests/test_narrow_constants.py checks every m and every dot.
 struct SkinnyConsts {
     uint32_t w[kMaxS][2], magic[kMaxS];
     int init[kMaxS], mneg[kMaxS];
@@ -292,6 +293,20 @@ int skinny_parts(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int 
     return 0;
 }
 
+NarrowModulus narrow_modulus(int m1) {
+    const int m = 255 / m1 * m1, h = m / 2;
+    NarrowModulus c{};
+    int p = 1;  // 256^j mod m, symmetric
+    for (int j = 0; j < 8; j++, p = p * 256 % m)
+        c.w[j / 4] |= (uint32_t)((p > h ? p - m : p) & 0xFF) << (8 * (j % 4));
+    int L = ((1 << 17) + m - 1) / m;
+    while ((2 * h + L * m) % 256) L++;
+    c.magic = m == 128 ? 0u : (uint32_t)(((1ull << 31) + m - 1) / m);
+    c.init = 2 * h + 2 * L * m;
+    c.mneg = (1 << 24) - m;
+    return c;
+}
+
 int launch_skinny(oz_dev* dev, const double* A, int M, int K, int lda, const int32_t* dA, const int8_t* pB, int Kg,
                   uint8_t* D, int ldd, long long sD, int parts, const oz2_moduli_dev* mo, const oz2_crt_dev* crt) {
     SkinnyConsts k{};
@@ -305,15 +320,12 @@ int launch_skinny(oz_dev* dev, const double* A, int M, int K, int lda, const int
             k.c1 = mo->c[1][s];
         }
     for (int i = 0; i < kMaxS; i++) {
-        const int m1 = (int)mo->m[std::min(i, mo->S - 1)], m = 255 / m1 * m1, h = m / 2;
-        int p = 1;  // 256^j mod m, symmetric
-        for (int j = 0; j < 8; j++, p = p * 256 % m)
-            k.w[i][j / 4] |= (uint32_t)((p > h ? p - m : p) & 0xFF) << (8 * (j % 4));
-        int L = ((1 << 17) + m - 1) / m;
-        while ((2 * h + L * m) % 256) L++;
-        k.magic[i] = (uint32_t)(((1ull << 31) + m - 1) / m);
-        k.init[i] = 2 * h + 2 * L * m;
-        k.mneg[i] = (1 << 24) - m;
+        const NarrowModulus c = narrow_modulus((int)mo->m[std::min(i, mo->S - 1)]);
+        k.w[i][0] = c.w[0];
+        k.w[i][1] = c.w[1];
+        k.magic[i] = c.magic;
+        k.init[i] = c.init;
+        k.mneg[i] = c.mneg;
     }
     oz2::DigitConsts dc{};
     for (int s = 0; s < mo->S; s++) {
