@@ -57,12 +57,15 @@ __global__ void __launch_bounds__(THREADS) gemm_f8_groups_kernel(const uint8_t* 
                                                                  const uint8_t* __restrict__ Bt, void* __restrict__ out,
                                                                  int K, int ldo, long long sA, long long sB,
                                                                  long long sO, int tiles_m, int tiles_n, int nout,
-                                                                 GroupArgs ga) {
+                                                                 int ranges, GroupArgs ga) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * STAGE];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int o, tm, tn;
-    tile_of_lockstep(blockIdx.x, tiles_m, tiles_n, nout, o, tm, tn);
+    if (ranges)
+        tile_of(blockIdx.x, tiles_m, tiles_n, nout, o, tm, tn);
+    else
+        tile_of_lockstep(blockIdx.x, tiles_m, tiles_n, nout, o, tm, tn);
     // wave-uniform: kept in SGPRs (the map divides on the VALU), so the output's constants come in
     // by scalar loads and every load address below stays on the SALU
     o = __builtin_amdgcn_readfirstlane(o);
@@ -289,9 +292,10 @@ extern "C" int oz2_gemm_groups_f8(oz_dev* dev, const uint8_t* A, const uint8_t* 
     const int tiles_m = M / BM, tiles_n = N / BN;
     const unsigned grid = (unsigned)((long long)tiles_m * tiles_n * gd->nout);
     const int nout = gd->nout;
+    const int ranges = grid <= (unsigned)dev->cus && tiles_m * tiles_n % 8 != 0;
 #define OZ_F8_LAUNCH(KIND, EVEN)                                                                                      \
     oz::launch_product(dev, gemm_f8_groups_kernel<KIND, EVEN>, dim3(grid), dim3(THREADS), A, Bt, out, K, ldo,     \
-                       strideA, strideB, strideO, tiles_m, tiles_n, nout, ga)
+                       strideA, strideB, strideO, tiles_m, tiles_n, nout, ranges, ga)
     const bool even = (K / BK) % 2 == 0;
     if (out_kind == 1) {
         if (even) OZ_F8_LAUNCH(1, true);

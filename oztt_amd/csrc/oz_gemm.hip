@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(THREADS) gemm_i8_kernel(const int8_t* __restri
                                                           void* __restrict__ C, int K, int ldc, long long sA,
                                                           long long sB, long long sC, int tiles_m, int tiles_n,
                                                           int nbatch, oz2::DigitConsts dc, int* __restrict__ queue,
-                                                          int first) {
+                                                          int first, int ranges) {
     __shared__ __attribute__((aligned(1024))) int8_t lds[NS * STAGE];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -98,15 +98,7 @@ __global__ void __launch_bounds__(THREADS) gemm_i8_kernel(const int8_t* __restri
         if (w < 0) return;
     }
     int batch, tm, tn;
-    // A launch of at most one tile per CU (no pool: first == total) runs in one wave, and each XCD
-    // takes one contiguous range of the batch-major tile sequence (tile_of): whole moduli when a
-    // modulus has at most a few tiles (C1: 16 tiles of 1024^2, two moduli per XCD), whose operand
-    // bands then stay in that XCD's L2 (0.0594 against 0.0683 ms for the whole C1 pass). Larger
-    // launches sweep the moduli in step over all XCDs (tile_of_lockstep), sharing each modulus's
-    // operands through the Infinity Cache. Where 8 divides the (equally long) products but not their tiles, a
-    // contiguous range is whole products per XCD at any size, and as fast or faster: 16 products of 81 tiles
-    // (2304^3, whole pass) 289 -> 284 us, 100 tiles (2560^3) 358 -> 353, 225 tiles (3840^3) 934 -> 930.
-    if (first >= total || (MODE != DIAG && tiles_m * tiles_n % 8 && nbatch % 8 == 0))
+    if (ranges)  // oz::tile_ranges
         tile_of(w, tiles_m, tiles_n, nbatch, batch, tm, tn);
     else
         tile_of_lockstep(w, tiles_m, tiles_n, nbatch, batch, tm, tn);
@@ -346,6 +338,27 @@ const char* check_gemm(const int8_t* A, const int8_t* Bt, const void* C, int M, 
     return nullptr;
 }
 
+}  // namespace
+
+// Whether each XCD takes one contiguous range of the batch-major sequence of 256 x 256 tiles (tile_of), or all XCDs
+// sweep the products in step (tile_of_lockstep), sharing each one's operands through the Infinity Cache.
+//   - A launch of at most one tile per CU runs in one wave: whole products per XCD where one has at most a few
+//     tiles (C1: 16 tiles of 1024^2, two per XCD), whose operand bands then stay in that XCD's L2 (0.0594 against
+//     0.0683 ms for the whole C1 pass).
+//   - Where 8 does not divide a product's tiles, ranges are the faster map, ranges against lockstep: 16 products of
+//     25 tiles (1280^2 x 2048) 54.7 against 61.6 us, 14 of 36 (1536^2 x 2048) 58.3 against 66.0, 20 of 36 84.8 against
+//     92.3, 12 of 121 (2816^2 x 2048) 167 against 168, 16 of 225 (3840^3) 735 against 744. Unless the
+//     operands of the eight products in progress are more than the Infinity Cache holds (256 MB; 2304^2 x 8192, 302 MB,
+//     15 products: 497 against 482; 3328^2 x 8192 1039 against 998; 4352^2 x 4096, 285 MB, 880 either way) and
+//     the products are not whole ones per XCD.
+bool oz::tile_ranges(int cus, int M, int N, int K, int batch) {
+    const long long per = (long long)(M / BM) * (N / BN), tiles = per * batch;
+    if (cus > 0 && tiles <= cus) return true;
+    return per % 8 && (batch % 8 == 0 || std::min(batch, 8) * ((long long)M + N) * K < 288ll << 20);
+}
+
+namespace {
+
 template <int MODE>
 int launch_gemm(oz_dev* dev, const int8_t* A, const int8_t* Bt, void* C, int M, int N, int K, int batch, int ldc,
                 long long strideA, long long strideB, long long strideC, const oz2::DigitConsts& dc) {
@@ -370,14 +383,15 @@ int launch_gemm(oz_dev* dev, const int8_t* A, const int8_t* Bt, void* C, int M, 
     // workgroups (these would start only when the first tiles end, and lengthen the launch).
     const bool one_wave = dev->cus > 0 && tiles <= dev->cus;
     const int first = one_wave ? (int)tiles : TilePool::first_of((int)tiles, MODE == DIAG ? 8 : 16);
+    const int ranges = MODE == DIAG ? one_wave : oz::tile_ranges(dev->cus, M, N, K, batch);
     const unsigned grid = one_wave ? (unsigned)tiles : (unsigned)(tiles + std::max<long long>(tiles / 8, 8));
     // K/64 even: every tile has an even number of K steps (DIAG: (d+1) K/64), no tail step
     if ((K / BK) % 2 == 0)
         oz::launch_product(dev, gemm_i8_kernel<MODE, true>, dim3(grid), dim3(THREADS), A, Bt, C, K, ldc, strideA,
-                           strideB, strideC, tiles_m, tiles_n, batch, dc, dev->queue, first);
+                           strideB, strideC, tiles_m, tiles_n, batch, dc, dev->queue, first, ranges);
     else
         oz::launch_product(dev, gemm_i8_kernel<MODE, false>, dim3(grid), dim3(THREADS), A, Bt, C, K, ldc, strideA,
-                           strideB, strideC, tiles_m, tiles_n, batch, dc, dev->queue, first);
+                           strideB, strideC, tiles_m, tiles_n, batch, dc, dev->queue, first, ranges);
     return oz::launch_check(dev, "gemm_i8_kernel");
 }
 

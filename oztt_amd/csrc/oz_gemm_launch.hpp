@@ -16,6 +16,9 @@ struct ProductArgs {
     oz2::DigitConsts dc;
 };
 
+// The order of the 256 x 256 tiles of products of equal length (oz_gemm.hip).
+bool tile_ranges(int cus, int M, int N, int K, int batch);
+
 enum class DigitTile { Tile256, Tile256x128, Tile128, Tile64, Split4, Split8 };
 DigitTile digit_tile(int cus, int M, int N, int K, int S);
 int launch_digit_tile(oz_dev* dev, DigitTile tile, const ProductArgs& a);  // not Tile256
