@@ -52,6 +52,9 @@ namespace oz {
 //   6144 (1536 x 1024)      29.0 -> 21.1         63.8 -> 49.4 (2048), 109 -> 89.4, 233 -> 194 (8192)
 //   16384 (2048 x 2048)     56.7 -> 51.0         76.7 -> 74.5 (1024); 231 against 262 (4096)
 //   36864 (3072 x 3072)     129 -> 112           188 -> 183 (1024)
+// and with other numbers of moduli, where 256 x 256 tiles fill more than three quarters of their rounds and K is long:
+//   6400 (1280^2, 16)       78 against 85 (3072), 185 against 211 (8192)
+//   6272 (1792^2, 8)        97 against 108 (4096), 178 against 202 (8192)
 DigitTile digit_tile(int cus, int M, int N, int K, int S) {
     const long long t64 = (long long)(M / 64) * (N / 64) * S, t256 = t64 / 16;
     if (cus <= 0 || t256 > (1 << 28)) return DigitTile::Tile256;
@@ -60,7 +63,7 @@ DigitTile digit_tile(int cus, int M, int N, int K, int S) {
         return t64 <= 6ll * cus || K <= (t64 <= 9ll * cus ? 2048 : 1024) ? DigitTile::Tile128 : DigitTile::Tile256;
     const long long rounds = (t256 + cus - 1) / cus;  // of the 256 x 256 tiles over the CUs
     if (rounds == 1) return K < 512 ? DigitTile::Tile256x128 : DigitTile::Tile256;
-    return K <= 1024 || 5 * t256 < 4 * rounds * cus ? DigitTile::Tile256x128 : DigitTile::Tile256;
+    return K <= 1024 || 4 * t256 <= 3 * rounds * cus ? DigitTile::Tile256x128 : DigitTile::Tile256;
 }
 
 int launch_digit_tile(oz_dev* dev, DigitTile tile, const ProductArgs& a) {

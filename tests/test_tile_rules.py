@@ -20,3 +20,19 @@ CUS = 256
 ])
 def test_order_of_the_large_tiles(M, N, K, batch, ranges):
     assert hip().oz_rule_tile_ranges(CUS, M, N, K, batch) == ranges
+
+
+TILE256, TILE256X128, TILE128, TILE64, SPLIT4, SPLIT8 = range(6)
+
+
+@pytest.mark.parametrize("M,N,K,S,tile", [
+    (256, 256, 512, 16, TILE64), (256, 256, 576, 16, SPLIT8), (512, 256, 576, 16, SPLIT4), (512, 512, 64, 16, TILE128),
+    (512, 512, 8192, 16, TILE128), (768, 768, 2048, 16, TILE128), (768, 768, 2112, 16, TILE256),
+    (1024, 768, 1024, 16, TILE128), (1024, 1024, 448, 16, TILE256X128), (1024, 1024, 512, 16, TILE256),
+    (2048, 2048, 1024, 16, TILE256X128), (2048, 2048, 1088, 16, TILE256),
+    (1536, 1024, 8192, 16, TILE256X128),                                # 384 large tiles: three quarters of two rounds
+    (1280, 1024, 2048, 20, TILE256), (1280, 1280, 8192, 16, TILE256), (1792, 1792, 4096, 8, TILE256),  # a little more
+    (2304, 2304, 3072, 5, TILE256), (2304, 2304, 1024, 5, TILE256X128),
+])
+def test_tiles_of_the_digits(M, N, K, S, tile):
+    assert hip().oz_rule_digit_tile(CUS, M, N, K, S) == tile
