@@ -83,15 +83,35 @@ int launch_digit_tile(oz_dev* dev, DigitTile tile, const ProductArgs& a) {
 //   512 (2048 x 1024)  59.8 -> 40.5 (512), 102 -> 69 (1024), 193 -> 125 (2048), 678 -> 494 (8192)
 //   1024 (2048 x 2048) 54.1 -> 43.5 (192), 77.7 -> 74.9 (512); 139 against 141 (1024)
 //   4096 (4096 x 4096) 204.6 -> 167.6 (192); 347 against 370 (512); 1742 against 1776 (4096)
+// With p slices the 256 x 256 tiles take n p (p + 1) / 2 steps of K (n tiles per diagonal) on `cus` CUs and at least
+// the p of the longest diagonal: `fill` of that is work. 128 x 128 tiles (times second) cost more per step and less
+// per tile, so they lose where the large ones fill their time or are long:
+//   fill .55-.6   1280^2, 11 slices: 21.1 against 27.5 (128), 811 against 863 (8192), 206 in place of 215 (2048)
+//   fill .65-.7   1280^2, 13 slices: 26.0 against 31.1 (128), 510 against 603 (4096), 1008 against 1311 (8192)
+//   fill .63-.95  1536^2, 8: 24.3 against 29.5 (192); 2048 x 1536, 7: 28.8 against 33.1 (256); 2304^2, 5: 38.9 against
+//                 41.6 (384); but 2048^2, 6: 33.7 against 32.5 (192)
+//   fill .72-1.0  2048 x 1024, 13: 81 against 89 (512), 1057 against 1494 (8192); 256 x 8192, 13: 1248 against 1783
+//   long tiles    3584^2 x 384: 339 against 375 (12 slices), 545 against 627 (16); 180 either way with 8
 DiagTile diag_tile(int cus, int M, int N, int K, int p) {
-    const long long t64 = (long long)(M / 64) * (N / 64);
+    const long long t64 = (long long)(M / 64) * (N / 64), t256 = t64 / 16;
     const bool all = p >= 5 && p <= 9;  // the slices for which the all-diagonals kernel is built
     if (cus <= 0 || t64 * p > (1 << 28)) return DiagTile::Tile256;
     if (16 * t64 <= cus) return DiagTile::Split32;
     if (2 * t64 < cus) return K <= 128 ? DiagTile::Tile64 : DiagTile::Split64;
-    if (t64 <= cus) return all && K >= 512 ? DiagTile::All : DiagTile::Tile128;
-    if (t64 <= 2ll * cus) return all && K >= 2048 ? DiagTile::All : DiagTile::Tile128;
-    return K <= 384 ? DiagTile::Tile128 : DiagTile::Tile256;
+    const int nk = K / BK;
+    const double fill = 0.5 * (double)t256 * (p + 1) / cus;
+    if (t64 <= 2ll * cus) {
+        if (all && K >= (t64 <= cus ? 512 : 2048)) return DiagTile::All;
+        const bool two = t64 == 2ll * cus;  // (2048 x 1024 x 128: 128 x 128 tiles up to 13% faster, 12 slices)
+        const double least = nk < 2 || (two && nk < 3) ? 2.0 : nk < 5 ? (two ? 0.62 : 0.54) : nk < 8 ? (two ? 0.62 : 0.72) :
+                             nk < 32 ? 0.72 : nk < 64 ? 0.65 : 0.57;
+        return fill >= least && fill <= (nk < 8 ? 1.0 : 1.1) ? DiagTile::Tile256 : DiagTile::Tile128;
+    }
+    if (K > 384) return DiagTile::Tile256;
+    // up to one and a half rounds of large tiles, which the shorter diagonals fill
+    if (fill >= 0.62 && fill <= (p == 3 ? 1.2 : 1.0) && t256 * p > cus && p > 2 && (nk >= 3 || (nk == 2 && p >= 8)))
+        return DiagTile::Tile256;
+    return nk * (p + 1) > (t64 > 7ll * cus ? 60 : 96) ? DiagTile::Tile256 : DiagTile::Tile128;
 }
 
 int launch_diag_tile(oz_dev* dev, DiagTile tile, const ProductArgs& a) {

@@ -36,3 +36,24 @@ TILE256, TILE256X128, TILE128, TILE64, SPLIT4, SPLIT8 = range(6)
 ])
 def test_tiles_of_the_digits(M, N, K, S, tile):
     assert hip().oz_rule_digit_tile(CUS, M, N, K, S) == tile
+
+
+DIAG256, ALL, DIAG128, DIAG64, SPLIT64, SPLIT32 = range(6)
+
+
+@pytest.mark.parametrize("M,N,K,p,tile", [
+    (256, 256, 512, 8, SPLIT32), (512, 512, 128, 8, DIAG64), (512, 512, 192, 8, SPLIT64),
+    (1024, 1024, 448, 8, DIAG128), (1024, 1024, 512, 8, ALL), (2048, 1024, 1984, 8, DIAG128), (2048, 1024, 2048, 8, ALL),
+    (2048, 2048, 192, 8, DIAG128), (2048, 2048, 448, 8, DIAG256), (4096, 4096, 384, 8, DIAG128),
+    # more slices than the all-diagonals kernel has, or fewer: by the share of their time that large tiles fill
+    (1024, 768, 8192, 10, DIAG128), (2048, 1024, 1024, 10, DIAG128), (2048, 1024, 8192, 4, DIAG128),
+    (2048, 1024, 512, 13, DIAG256), (2048, 1024, 8192, 11, DIAG256), (256, 8192, 8192, 13, DIAG256),
+    (2048, 1024, 4096, 16, DIAG256), (2048, 1024, 128, 12, DIAG128), (256, 8192, 256, 16, DIAG128),
+    (1280, 1280, 128, 11, DIAG256), (1280, 1280, 1024, 11, DIAG128), (1280, 1280, 8192, 11, DIAG256),
+    (1280, 1280, 4096, 13, DIAG256), (1536, 1024, 8192, 16, DIAG256), (1536, 1024, 8192, 10, DIAG128),
+    (1536, 1536, 192, 8, DIAG256), (2048, 1536, 256, 7, DIAG256), (2304, 2304, 384, 5, DIAG256),
+    (2048, 2048, 256, 4, DIAG128), (2816, 2816, 384, 2, DIAG128), (3072, 3072, 384, 3, DIAG256),
+    (3584, 3584, 384, 12, DIAG256), (4096, 4096, 384, 16, DIAG256), (2048, 2048, 384, 10, DIAG128),
+])
+def test_tiles_of_the_diagonals(M, N, K, p, tile):
+    assert hip().oz_rule_diag_tile(CUS, M, N, K, p) == tile
