@@ -160,8 +160,9 @@ __global__ void __launch_bounds__(1024, 8) scale_pair_kernel(const double* __res
         const int r1 = CHUNKED ? min(K, r0 + chunk_rows) : K;
         const int col = strip * W + (t % W);
         const int ph = r0 + t / W;
-        // 16 loads in flight per thread (16 P rows of the strip per round trip)
-        uint32_t k[4] = {0, 0, 0, 0};
+        // 16 loads in flight per thread (16 P rows of the strip per round trip); two maxima, since with four
+        // CHUNKED spills in its 64 registers (256 x 256 x 2048 6.5 -> 6.2 us)
+        uint32_t k[2] = {0, 0};
         if (col < N) {
             const double* p = B + col;
             int r = ph;
@@ -170,18 +171,18 @@ __global__ void __launch_bounds__(1024, 8) scale_pair_kernel(const double* __res
 #pragma unroll
                 for (int u = 0; u < 16; u++) v[u] = p[(size_t)(r + P * u) * ldb];
 #pragma unroll
-                for (int u = 0; u < 16; u++) k[u & 3] = max(k[u & 3], bf16_key<CEIL>(v[u]));
+                for (int u = 0; u < 16; u++) k[u & 1] = max(k[u & 1], bf16_key<CEIL>(v[u]));
             }
             for (; r + 3 * P < r1; r += 4 * P) {
                 double v[4];
 #pragma unroll
                 for (int u = 0; u < 4; u++) v[u] = p[(size_t)(r + P * u) * ldb];
 #pragma unroll
-                for (int u = 0; u < 4; u++) k[u] = max(k[u], bf16_key<CEIL>(v[u]));
+                for (int u = 0; u < 4; u++) k[u & 1] = max(k[u & 1], bf16_key<CEIL>(v[u]));
             }
             for (; r < r1; r += P) k[0] = max(k[0], bf16_key<CEIL>(p[(size_t)r * ldb]));
         }
-        part[t] = max(max(k[0], k[1]), max(k[2], k[3]));  // part[W ph + c]
+        part[t] = max(k[0], k[1]);  // part[W ph + c]
         __syncthreads();
         // P phases per column: 8 threads per column take P/8 phases each, then one thread 8 of those
         uint32_t m8 = 0;

@@ -26,3 +26,16 @@ def test_m0_and_spills(src, tmp_path):
     meta = re.findall(r"\.name:\s+(_Z\S*" + SOURCES[src] + r"\S*)\s.*?\.private_segment_fixed_size:\s+(\d+).*?"
                       r"\.vgpr_spill_count:\s+(\d+)", asm, re.S)
     assert meta and all(p == "0" and s == "0" for _, p, s in meta), meta
+
+
+@pytest.mark.parametrize("src,stem", [("oz_scale.hip", "scale_pair_kernel"), ("oz2_prep.hip", "prep_kernel"),
+                                      ("oz2_split.hip", "split_"), ("oz2_crt.hip", "crt_digits_kernel")])
+def test_no_spills(src, stem, tmp_path):
+    # kernels whose registers are held down by launch bounds, or close to a step of the occupancy
+    out = tmp_path / "x.s"
+    cmd = [B.HIPCC, *B.HIP_FLAGS, *B.HIP_SOURCES[src], "--cuda-device-only", "-S", str(B.CSRC / src), "-o", str(out)]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    meta = re.findall(r"\.name:\s+(_Z\S*" + stem + r"\S*)\s.*?\.private_segment_fixed_size:\s+(\d+).*?"
+                      r"\.vgpr_spill_count:\s+(\d+)", out.read_text(), re.S)
+    assert meta and all(p == "0" and s == "0" for _, p, s in meta), meta
