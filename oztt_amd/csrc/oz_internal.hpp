@@ -73,6 +73,9 @@ inline int use(oz_dev* dev) {
     return hip_check(dev, hipSetDevice(dev->device), "hipSetDevice");
 }
 
+// Runs that oz_scale_pair_f64 cuts a strip of B's columns into (oz_scale.hip), and their rows.
+int strip_chunks(int cus, int M, int N, int K, int* chunk_rows);
+
 inline unsigned ceil_div(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
 
 }  // namespace oz

@@ -12,3 +12,7 @@ extern "C" void oz_rule_narrow_modulus(int m, oz2pass::NarrowModulus* out) { *ou
 extern "C" int oz_rule_digit_tile(int cus, int M, int N, int K, int S) { return (int)oz::digit_tile(cus, M, N, K, S); }
 extern "C" int oz_rule_diag_tile(int cus, int M, int N, int K, int p) { return (int)oz::diag_tile(cus, M, N, K, p); }
 extern "C" int oz_rule_tile_ranges(int cus, int M, int N, int K, int batch) { return oz::tile_ranges(cus, M, N, K, batch); }
+extern "C" int oz_rule_strip_chunks(int cus, int M, int N, int K) {
+    int rows;
+    return oz::strip_chunks(cus, M, N, K, &rows);
+}

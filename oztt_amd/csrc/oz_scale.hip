@@ -256,6 +256,32 @@ extern "C" int oz_scale_f64(oz_dev* dev, const double* X, int rows, int cols, in
     return oz::launch_check(dev, "key_to_delta_kernel");
 }
 
+// Runs of a strip of B's columns (32 wide, K > 1024): as many as give every CU two, of at least 512 rows (one round of
+// 16 loads per thread); 1 where that does not pay. A whole strip takes about 2.5 us + 4.4 ns K; beside it A's
+// rows (5 TB/s, say) fill the chip. Whole strips -> chunks, us, (M x N x K):
+//   K < 2048    64 x 2048 x 1100 8.0 -> 6.2, 1024^2 x 1100 8.2 -> 6.3, 16 x 2500 x 1200 9.4 -> 6.9: while both operands take less
+//               than a strip (2048^2 x 1025 8.2 against 8.8, 2048 x 2500 x 1200 11.2 against 12.6), up to 80 strips
+//               (512 x 3000 x 1025, 94 strips, 7.9 against 8.6)
+//   <= 8 strips 4096 x 64 x 2048 16.0 -> 13.7, 8192 x 64 x 8192 96 -> 87, 16384 x 256 x 3072 101 -> 96
+//   <= 64       2048^2 x 4096 28.4 -> 23.0, 4096 x 1024 x 4096 32.7 -> 27.3 (x 6144 41.5 against 43.6); 8192 x 1024 x 8192 98
+//               against 104
+//   <= 120      2048 x 3000 x 8192 70 -> 57; 4096 x 3000 x 3072 30.5 against 33.1
+//   more        16 x 4096 x 2048 13.9 against 15.1, 4096^3 39.9 against 42.0, 2048 x 4096 x 6144 49.5 against 56.5
+int oz::strip_chunks(int cus, int M, int N, int K, int* chunk_rows) {
+    const int strips = (N - 1) / 32 + 1;
+    *chunk_rows = K;
+    if (K <= 1024 || 2ll * strips > cus || strips > oz_dev::kStrips) return 1;
+    const double strip = 2.5 + 0.0044 * K, rows = 1.6e-6 * M * K, both = rows + 1.6e-6 * N * K;
+    const bool pays = K < 2048             ? strips <= 5 * cus / 16 && both < 0.9 * strip
+                      : strips <= cus / 4  ? strips <= 8 || rows < 1.5 * strip
+                      : strips <= 15 * cus / 32 ? rows < 0.75 * strip
+                                           : K >= 3072 && rows < 0.5 * strip;
+    if (!pays) return 1;
+    const int want = std::max(1, std::min((int)(((long long)K + 511) / 512), (2 * cus + strips - 1) / strips));
+    *chunk_rows = (int)((((long long)K + want - 1) / want + 511) / 512 * 512);
+    return (int)(((long long)K + *chunk_rows - 1) / *chunk_rows);
+}
+
 extern "C" int oz_scale_pair_f64(oz_dev* dev, const double* A, int M, int K, int lda, const double* B, int N, int ldb,
                                  int ceil_mode, int shift, int32_t* dA, int32_t* dB, uint32_t* flags,
                                  uint32_t* clear_flags) {
@@ -268,14 +294,9 @@ extern "C" int oz_scale_pair_f64(oz_dev* dev, const double* A, int M, int K, int
     int R = 1;  // rows of A per workgroup: 8 loads per thread for K <= 8192
     while (R < 16 && (long long)K * R * 2 <= 8192) R *= 2;
     const int W = K <= 1024 ? 16 : 32;  // columns of B per workgroup
-    // chunks of a strip: at least 512 rows (one round of 16 loads per thread), as many as give every CU two
     const int strips = (N + W - 1) / W;
-    int chunks = 1, chunk_rows = K;
-    if (W == 32 && 2 * strips <= dev->cus && strips <= oz_dev::kStrips) {
-        chunks = std::max(1, std::min((K + 511) / 512, (2 * dev->cus + strips - 1) / strips));
-        chunk_rows = ((K + chunks - 1) / chunks + 511) / 512 * 512;
-        chunks = (K + chunk_rows - 1) / chunk_rows;
-    }
+    int chunk_rows = K;
+    const int chunks = oz::strip_chunks(dev->cus, M, N, K, &chunk_rows);
     const long long blocks = ((long long)M + R - 1) / R + (long long)strips * chunks;
     if (blocks > 0x7FFFFFFFll) return oz::fail(dev, OZ_ERR_ARG, "oz_scale_pair_f64: grid too large");
     const dim3 grid((unsigned)blocks), block(1024);

@@ -7,7 +7,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N,K", [(1, 1025), (31, 1536), (33, 1537), (32, 2050), (65, 9001), (4096, 1100), (12, 33000)])
+@pytest.mark.parametrize("N,K", [(1, 1025), (31, 1536), (33, 1537), (32, 2050), (65, 9001), (4096, 1100), (12, 33000), (4077, 3100),
+                                 (2499, 1300)])
 def test_chunked_columns_match_oracle(dev, oracle, N, K):
     M, lda, ldb, shift = 9, K + 2, N + 3, 16
     rng = np.random.default_rng(N + K)

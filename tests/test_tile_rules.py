@@ -1,5 +1,5 @@
-"""The rules by which a launch of INT8 products takes its tiles and their order (oz_gemm_tiles.hip, oz_gemm.hip), at
-sizes on either side of their lines, on 256 compute units. Every choice was measured against the others at the size
+"""The rules by which a launch of INT8 products takes its tiles and their order (oz_gemm_tiles.hip, oz_gemm.hip), and the
+scale cuts strips of columns (oz_scale.hip), at sizes on either side of their lines, on 256 compute units. Every choice was measured against the others at the size
 given. CPU only: the library's own rules are asked."""
 import pytest
 
@@ -57,3 +57,14 @@ DIAG256, ALL, DIAG128, DIAG64, SPLIT64, SPLIT32 = range(6)
 ])
 def test_tiles_of_the_diagonals(M, N, K, p, tile):
     assert hip().oz_rule_diag_tile(CUS, M, N, K, p) == tile
+
+
+@pytest.mark.parametrize("M,N,K,cut", [
+    (64, 2048, 1024, False), (256, 256, 1025, True), (64, 2048, 1100, True), (2048, 2048, 1025, False), (16, 2500, 1200, True),
+    (2048, 2500, 1200, False), (512, 3000, 1025, False), (16, 4096, 2048, False), (16, 4096, 4096, True),
+    (2048, 2048, 4096, True), (4096, 4096, 4096, False), (8192, 64, 8192, True), (8192, 1024, 8192, False),
+    (4096, 1024, 4096, True), (2048, 3000, 8192, True), (4096, 3000, 3072, False), (256, 256, 32768, True),
+    (64, 4097, 32768, False),
+])
+def test_strips_that_the_scale_cuts(M, N, K, cut):
+    assert (hip().oz_rule_strip_chunks(CUS, M, N, K) > 1) == cut
