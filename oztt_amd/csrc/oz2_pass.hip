@@ -101,7 +101,7 @@ int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, do
     const long long sB = (long long)L.Ng * L.Kg;
     const bool fused = fused_reconstruction(dev, M, N, L.Kg, crt);
     // a matrix on at most 64 columns: B's planes only (64 rows of them)
-    const int parts = skinny_parts(dev, mo, M, N, K);
+    const int parts = skinny_parts(dev->cus, mo, M, N, K);
     if (parts) {
         if (int st = oz_scale_pair_f64(dev, A, M, K, lda, B, N, ldb, 1, crt->shift, dA, dB, collect, nullptr)) return st;
         if (int st = oz2_split_int8(dev, B, K, N, ldb, 1, dB, mo, pB, 3, 64, L.Kg, 64ll * L.Kg)) return st;

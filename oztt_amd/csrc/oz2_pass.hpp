@@ -59,7 +59,7 @@ struct NarrowModulus {
     int init, mneg;
 };
 NarrowModulus narrow_modulus(int m1);
-int skinny_parts(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int K);
+int skinny_parts(int cus, const oz2_moduli_dev* mo, int M, int N, int K);
 int launch_skinny(oz_dev* dev, const double* A, int M, int K, int lda, const int32_t* dA, const int8_t* pB, int Kg,
                   uint8_t* D, int ldd, long long sD, int parts, const oz2_moduli_dev* mo, const oz2_crt_dev* crt);
 

@@ -280,15 +280,20 @@ namespace oz2pass {
 
 // The parts of K (0: the kernel does not take the pass). It takes three digits and at most 16 moduli, and pays
 // from where normalization and residues are no longer one launch (K > 512, oz2_prep.hip) and its workgroups, one
-// per CU, fill the chip: with 192 of them (M = 6144, two parts) the pass takes 77 us against 95 at K = 1024.
-int skinny_parts(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int K) {
+// per CU, fill the chip: with 192 of them (M = 6144, two parts) the pass takes 77 us against 95 at K = 1024. And from a
+// number of moduli on, whose planes are what it saves while it makes A' and the matrix products of at least 8 (with
+// planes -> here, 64 columns): 8192 x 1024 with 3 moduli 58 against 56 us, with 2 53 against 55, x 2048 89 against 87
+// and 79 against 85; with three quarters of the CUs 6144 x 2048 with 6 94 -> 84, with 5 82 either way, with 4 79 against 82, 12288
+// x 2048 with 5 136 against 145.
+int skinny_parts(int cus, const oz2_moduli_dev* mo, int M, int N, int K) {
     int evens = 0;  // (more than one, and the planes are all of the sequence on the digits)
     for (int s = 0; s < mo->S; s++) evens += (int)mo->m[s] % 2 == 0;
-    if (N > 64 || mo->nd != 3 || mo->S > kMaxS || K < 1024 || evens > 1) return 0;
-    const long long groups = (M + 63ll) / 64, cus = dev->cus;
+    if (N > 64 || mo->nd != 3 || mo->S < 4 || mo->S > kMaxS || K < 1024 || evens > 1) return 0;
+    const long long groups = (M + 63ll) / 64;
     for (int parts = 1; parts <= 2; parts++) {
         const long long w = groups * parts, rounds = (w + cus - 1) / cus;
-        if (4 * w >= 3 * rounds * cus) return parts;  // at least three quarters of the CUs in every round
+        if (4 * w >= 3 * rounds * cus)  // at least three quarters of the CUs in every round
+            return mo->S >= 6 || 10 * w >= 9 * rounds * cus ? parts : 0;
     }
     return 0;
 }

@@ -16,3 +16,6 @@ extern "C" int oz_rule_strip_chunks(int cus, int M, int N, int K) {
     int rows;
     return oz::strip_chunks(cus, M, N, K, &rows);
 }
+extern "C" int oz_rule_narrow_parts(int cus, const oz2_moduli_dev* mo, int M, int N, int K) {
+    return oz2pass::skinny_parts(cus, mo, M, N, K);
+}

@@ -83,6 +83,7 @@ def test_range_flags(dev):
     (100, 90, 120, 0, None), (300, 4000, 512, 0, None), (300, 300, 700, 0, None), (1500, 1409, 64, 0, None),
     (6100, 20, 1030, 0, None), (12290, 64, 1100, 0, None), (6081, 64, 1999, 0, None), (6100, 33, 1024, 30, None),
     (6144, 17, 1100, 0, [255, 253, 251, 247, 2, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193]),
+    (8192, 24, 1100, 0, [255, 254, 253, 251]),
     (6144, 9, 1100, 0, [255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193]),
 ])
 def test_flagged_operands_equal_the_stages(dev, M, N, K, width, moduli):
