@@ -128,7 +128,7 @@ __device__ __forceinline__ double finish(double* x, const FusedCrt<L>& a, int e2
     const double r0 = fix ? __builtin_fma(2.0, h, s) : s;
     const int ex = ((__double2hiint(r0) >> 20) & 0x7FF) - 1023 + e2;
     double r = __builtin_ldexp(r0, e2);
-    r = ex < -1022 ? 0.0 : r;
+    r = ex < -1022 ? 0.0 : r;  // (only by a b far from any plan's: e2 >= -252 - 2 b, and C' = 0 for smaller maxima)
     r = neg ? -r : r;
     return r0 == 0.0 ? 0.0 : r;
 }

@@ -69,10 +69,19 @@ const char* check_plan(const oz2_moduli_dev* mo, const oz2_crt_dev* crt, int Kg)
 //   4096 x 4096: 211 -> 147 (K 64), 222 -> 173 (128), 266 -> 226 (256), 350 against 333 (512, where the
 //   8192 x 8192 result takes 1241 against 1290); 2048 x 2048: 78 -> 64 (128), 86 -> 78 (256), 104 against
 //   107 (512); 1024 x 1024 (one tile per CU): 38 -> 36 (64), 41 against 44 (256).
-static bool fused_reconstruction(const oz_dev* dev, int M, int N, int Kg, const oz2_crt_dev* crt) {
+static bool fused_reconstruction(int cus, int M, int N, int Kg, const oz2_crt_dev* crt) {
     const long long tiles = ((M + 63ll) / 64) * ((N + 63ll) / 64);
     int width, limbs;
-    return Kg <= 256 && tiles >= 2ll * dev->cus && tiles <= 0x7FFFFFFFll && oz::fused_limbs(crt, Kg, &width, &limbs);
+    return Kg <= 256 && tiles >= 2ll * cus && tiles <= 0x7FFFFFFFll && oz::fused_limbs(crt, Kg, &width, &limbs);
+}
+
+Route route_of(int cus, const oz2_moduli_dev* mo, const oz2_crt_dev* crt, int M, int N, int K) {
+    const int Kg = (K + 63) / 64 * 64;
+    Route r{};
+    r.parts = skinny_parts(cus, mo, M, N, K);
+    r.prep = !r.parts && prep_takes(cus, mo, M, N, Kg);
+    r.fused = !r.parts && fused_reconstruction(cus, M, N, Kg, crt);
+    return r;
 }
 
 int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, double* C, int ldc, int M, int N, int K,
@@ -99,13 +108,13 @@ int run_pass(oz_dev* dev, const double* A, int lda, const double* B, int ldb, do
         }
     } failed{dev, collect, flags, true};
     const long long sB = (long long)L.Ng * L.Kg;
-    const bool fused = fused_reconstruction(dev, M, N, L.Kg, crt);
-    // a matrix on at most 64 columns: B's planes only (64 rows of them)
-    const int parts = skinny_parts(dev->cus, mo, M, N, K);
-    if (parts) {
+    const Route route = route_of(dev->cus, mo, crt, M, N, K);
+    const int parts = route.parts;
+    const bool fused = route.fused;
+    if (parts) {  // B's planes only (64 rows of them)
         if (int st = oz_scale_pair_f64(dev, A, M, K, lda, B, N, ldb, 1, crt->shift, dA, dB, collect, nullptr)) return st;
         if (int st = oz2_split_int8(dev, B, K, N, ldb, 1, dB, mo, pB, 3, 64, L.Kg, 64ll * L.Kg)) return st;
-    } else if (prep_takes(dev, mo, M, N, L.Kg)) {
+    } else if (route.prep) {
         // the fused kernel reads rows up to a multiple of 64 only
         const int Mt = fused ? (M + 63) / 64 * 64 : L.Mg, Nt = fused ? (N + 63) / 64 * 64 : L.Ng;
         const PrepArgs p{A,  M, K,   lda, Mt, dA, reinterpret_cast<uint8_t*>(pA), sA,         B,

@@ -46,7 +46,7 @@ struct PrepArgs {
     int Kg, shift;
     uint32_t* flags;
 };
-bool prep_takes(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int Kg);
+bool prep_takes(int cus, const oz2_moduli_dev* mo, int M, int N, int Kg);
 int launch_prep(oz_dev* dev, const PrepArgs& a, const oz2_moduli_dev* mo);
 
 // A matrix on at most 64 columns (oz2_skinny.hip): the digits of A's products with B's residue planes (64 rows
@@ -62,5 +62,13 @@ NarrowModulus narrow_modulus(int m1);
 int skinny_parts(int cus, const oz2_moduli_dev* mo, int M, int N, int K);
 int launch_skinny(oz_dev* dev, const double* A, int M, int K, int lda, const int32_t* dA, const int8_t* pB, int Kg,
                   uint8_t* D, int ldd, long long sD, int parts, const oz2_moduli_dev* mo, const oz2_crt_dev* crt);
+
+// The way of a pass: the parts of K without A's planes (0: with planes), else normalization and residues in one
+// launch or two, products and reconstruction in one kernel or two.
+struct Route {
+    int parts;
+    bool prep, fused;
+};
+Route route_of(int cus, const oz2_moduli_dev* mo, const oz2_crt_dev* crt, int M, int N, int K);
 
 }  // namespace oz2pass

@@ -113,11 +113,11 @@ namespace oz2pass {
 // 4096 x 4096 x 512 337 -> 305; 8192 x 8192 x 512 1195 -> 1126; 512^3 34.1 against 35.5; 8192 x 64 x 512
 // 81.2 against 83.5. At K = 1024 16 elements per lane leave one workgroup per CU, nothing hides its loads,
 // and 272 bands take two rounds: 79 against 102 (4096 x 256 x 1024).
-bool prep_takes(const oz_dev* dev, const oz2_moduli_dev* mo, int M, int N, int Kg) {
+bool prep_takes(int cus, const oz2_moduli_dev* mo, int M, int N, int Kg) {
     int evens = 0;
     for (int s = 0; s < mo->S; s++) evens += (int)mo->m[s] % 2 == 0;
     if (evens > 1) return false;
-    return Kg <= 256 || (Kg <= 512 && mo->nd == 3 && M >= 256 && N >= 256 && ((long long)M + N) / 16 >= dev->cus);
+    return Kg <= 256 || (Kg <= 512 && mo->nd == 3 && M >= 256 && N >= 256 && ((long long)M + N) / 16 >= cus);
 }
 
 int launch_prep(oz_dev* dev, const PrepArgs& a, const oz2_moduli_dev* mo) {

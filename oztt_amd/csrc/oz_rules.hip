@@ -16,6 +16,8 @@ extern "C" int oz_rule_strip_chunks(int cus, int M, int N, int K) {
     int rows;
     return oz::strip_chunks(cus, M, N, K, &rows);
 }
-extern "C" int oz_rule_narrow_parts(int cus, const oz2_moduli_dev* mo, int M, int N, int K) {
-    return oz2pass::skinny_parts(cus, mo, M, N, K);
+// 4 parts + 2 fused + prep
+extern "C" int oz_rule_pass(int cus, const oz2_moduli_dev* mo, const oz2_crt_dev* crt, int M, int N, int K) {
+    const oz2pass::Route r = oz2pass::route_of(cus, mo, crt, M, N, K);
+    return 4 * r.parts + 2 * r.fused + r.prep;
 }

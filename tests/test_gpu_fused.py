@@ -2,11 +2,13 @@
 (checked against the oracle elsewhere), bit for bit: products and reconstruction in one kernel
 (oz2_gemm_crt.hip: short K, large results), normalization and residues in one (oz2_prep.hip: short K),
 and the range flags that the last kernel hands over."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import oztt_amd as oz
-from oztt_amd.device import crt_desc, moduli_desc
+from oztt_amd.device import crt_desc, hip, moduli_desc
 
 pytestmark = pytest.mark.gpu
 
@@ -22,18 +24,26 @@ def operands(M, N, K, seed, phi):
     A[4] = np.abs(A[4]) + 1e-3      # parallel to column 5: sums near the bound
     B[:, 5] = A[4]
     A[6] = -A[4]
-    A[7] *= 2.0 ** -600             # results below the normal range once multiplied
+    A[7] *= 2.0 ** -600             # maxima below the range: a flag, no digits, zeros
     B[:, 8] *= 2.0 ** -500
+    if M > 9:
+        A[8] *= 2.0 ** -125 / np.abs(A[8]).max()   # the smallest exponents that results have (2^-252 and less)
+    if N > 9:
+        B[:, 9] *= 2.0 ** -125 / np.abs(B[:, 9]).max()
     return A, B
+
+
+PREP, FUSED, PART = 1, 2, 4  # ways of a pass (oz_rules.hip)
 
 
 @pytest.mark.parametrize("M,N,K,phi,width", [
     (1500, 1409, 64, 0.5, 0), (2048, 1024, 128, 0.5, 0), (1473, 1472, 250, 1.0, 0), (1440, 1473, 193, 2.0, 0),
     (700, 3300, 1, 0.5, 0), (1500, 1409, 256, 0.5, 30), (1500, 1409, 256, 4.0, 60), (1500, 1409, 256, 0.5, 66),
+    (1409, 1500, 100, 2.0, 70),
 ])
 def test_fused_pass_equals_the_stages(dev, M, N, K, phi, width):
     A, B = operands(M, N, K, M + K, phi)
-    pass_equals_stages(dev, A, B, M, N, K, width)
+    assert pass_equals_stages(dev, A, B, M, N, K, width) == PREP | FUSED
 
 
 # deltas and planes in one launch (oz2_prep.hip): 4 elements per lane up to K = 256, 8 up to 512, bands and
@@ -41,21 +51,25 @@ def test_fused_pass_equals_the_stages(dev, M, N, K, phi, width):
 @pytest.mark.parametrize("M,N,K,width", [
     (9, 9, 1, 0), (17, 33, 64, 0), (100, 60, 33, 0), (128, 128, 128, 0), (300, 65, 256, 66), (40, 31, 200, 84),
     (256, 4000, 512, 0), (3900, 300, 449, 0), (2048, 2049, 300, 30),
+    (70, 90, 256, 86), (9, 17, 1, 80),
 ])
 def test_prepared_pass_equals_the_stages(dev, M, N, K, width):
     A, B = operands(M, N, K, M + K, 1.0)
-    pass_equals_stages(dev, A, B, M, N, K, width)
+    assert pass_equals_stages(dev, A, B, M, N, K, width) & PREP
 
 
 # at most 64 columns (oz2_skinny.hip): K in one part and in two, uneven halves, ragged rows, columns and K,
-# elements in 16-byte pairs (odd K here) and single ones, few moduli, and 17 of them (not taken)
+# elements in 16-byte pairs (odd K here) and single ones, few moduli, and 17 of them and more (not taken)
 @pytest.mark.parametrize("M,N,K,phi,width", [
     (6081, 64, 1024, 0.5, 0), (6100, 9, 1089, 1.0, 0), (8191, 33, 1027, 2.0, 0), (12290, 61, 1100, 0.5, 0),
     (12225, 64, 1025, 0.5, 30), (6144, 64, 1152, 0.5, 40), (6081, 63, 1999, 4.0, 0), (6144, 17, 1024, 0.5, 66),
+    (8191, 33, 1027, 0.5, 0), (6081, 63, 1999, 0.5, 0),
 ])
 def test_narrow_pass_equals_the_stages(dev, M, N, K, phi, width):
     A, B = operands(M, N, K, M + K, phi)
-    pass_equals_stages(dev, A, B, M, N, K, width)
+    # (17 moduli by the spread of the elements, and by the width)
+    taken = width != 66 and phi not in (2.0, 4.0)
+    assert pass_equals_stages(dev, A, B, M, N, K, width) // PART == (0 if not taken else 1 if M > 12224 else 2)
 
 
 def test_range_flags(dev):
@@ -81,7 +95,7 @@ def test_range_flags(dev):
 # the narrow one both parts of K, few moduli, and 2 as the even one.
 @pytest.mark.parametrize("M,N,K,width,moduli", [
     (100, 90, 120, 0, None), (300, 4000, 512, 0, None), (300, 300, 700, 0, None), (1500, 1409, 64, 0, None),
-    (6100, 20, 1030, 0, None), (12290, 64, 1100, 0, None), (6081, 64, 1999, 0, None), (6100, 33, 1024, 30, None),
+    (1500, 1409, 200, 66, None), (300, 65, 256, 84, None), (6100, 20, 1030, 0, None), (12290, 64, 1100, 0, None), (6081, 64, 1999, 0, None), (6100, 33, 1024, 30, None),
     (6144, 17, 1100, 0, [255, 253, 251, 247, 2, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193]),
     (8192, 24, 1100, 0, [255, 254, 253, 251]),
     (6144, 9, 1100, 0, [255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193]),
@@ -101,15 +115,22 @@ def test_flagged_operands_equal_the_stages(dev, M, N, K, width, moduli):
         X[13] = 2.0 ** -1060
         X[15, n - 1] = 2.0 ** 128
     A[M - 1, K - 1] = np.nan
-    pass_equals_stages(dev, A, B, M, N, K, width, operands(M, N, K, 1, 0.5), moduli=moduli)
+    way = pass_equals_stages(dev, A, B, M, N, K, width, operands(M, N, K, 1, 0.5), moduli=moduli)
+    assert way == (PREP | FUSED if M == 1500 else PREP if K <= 512 else 0 if M == 300 else PART if M > 12224 else 2 * PART)
 
 
 def pass_equals_stages(dev, A, B, M, N, K, width, plan=None, want_flags=None, moduli=None):
+    # width 0: the plan; up to 60 bits: the plan at that width; above: the moduli for it, in four or five digits (the
+    # planner stops at 16 moduli)
     PA, PB = plan or (A, B)
-    p = oz.plan2_int8(PA.ravel(), PB.ravel(), M, N, K, fixed_bits=width)
+    if width > 60:
+        p, b, nd = oz.choose_moduli_int8(K, 24, width), width, -(-width // 20)
+    else:
+        p = oz.plan2_int8(PA.ravel(), PB.ravel(), M, N, K, fixed_bits=width)
+        b, nd = p.b, p.nd
     moduli = moduli or [p.m[i] for i in range(p.S)]
     S = len(moduli)
-    md, cd = moduli_desc(moduli, p.nd), crt_desc(moduli, p.b, p.nd)
+    md, cd = moduli_desc(moduli, nd), crt_desc(moduli, b, nd)
     lda, ldb, ldc = K + 3, N + 5, N + 7
     a, b = np.zeros((M, lda)), np.zeros((K, ldb))
     a[:, :K], b[:, :N] = A, B
@@ -140,3 +161,4 @@ def pass_equals_stages(dev, A, B, M, N, K, width, plan=None, want_flags=None, mo
     for x in (bA, bB, bC, fl, work, dA, dB, f2, pA, pB, dg, out):
         x.free()
     dev.bufs.clear()
+    return hip().oz_rule_pass(256, ctypes.byref(md), ctypes.byref(cd), M, N, K)

@@ -4,6 +4,8 @@ different runs; twice, since the last run clears what the strip used."""
 import numpy as np
 import pytest
 
+from oztt_amd.device import hip
+
 pytestmark = pytest.mark.gpu
 
 
@@ -11,6 +13,7 @@ pytestmark = pytest.mark.gpu
                                  (2499, 1300)])
 def test_chunked_columns_match_oracle(dev, oracle, N, K):
     M, lda, ldb, shift = 9, K + 2, N + 3, 16
+    assert (hip().oz_rule_strip_chunks(256, M, N, K) > 1) == ((N, K) != (4096, 1100))  # (whole strips there)
     rng = np.random.default_rng(N + K)
     A = np.full((M, lda), 1e300)
     A[:, :K] = rng.uniform(-1, 1, (M, K))

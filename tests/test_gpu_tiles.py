@@ -5,11 +5,11 @@ The reference is the product in float64 (BLAS), which is exact: every sum is an 
 import numpy as np
 import pytest
 
-from oztt_amd.device import crt_desc, to_blocks
+from oztt_amd.device import crt_desc, hip, to_blocks
 
 pytestmark = pytest.mark.gpu
 
-MODULI = [255, 254, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193]
+MODULI = [255, 254, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193, 191, 181, 179, 173, 167, 163, 157, 151]
 
 
 def planes(rng, S, R, K):
@@ -19,14 +19,20 @@ def planes(rng, S, R, K):
     return X
 
 
-@pytest.mark.parametrize("M,N,K,S", [
-    (256, 256, 64, 1), (256, 256, 512, 16), (512, 256, 192, 16),      # 64 x 64
-    (256, 256, 576, 16), (256, 256, 1088, 3),                         # 64 x 64, K over 8 waves
-    (512, 256, 576, 16),                                              # ... over 4 waves
-    (512, 512, 64, 16), (768, 768, 128, 16), (512, 768, 576, 13),     # 128 x 128
-    (1024, 1024, 448, 16), (1536, 1024, 64, 16), (256, 6656, 192, 16),  # 256 x 128
+# The tile that each size stands for is asked of the rule (256 compute units).
+TILE256, TILE256X128, TILE128, TILE64, SPLIT4, SPLIT8 = range(6)
+
+
+@pytest.mark.parametrize("tile,M,N,K,S", [
+    (TILE64, 256, 256, 64, 1), (TILE64, 256, 256, 512, 16), (TILE64, 512, 256, 192, 16),
+    (SPLIT8, 256, 256, 576, 16), (SPLIT8, 256, 256, 1088, 3),         # 64 x 64, K over 8 waves
+    (SPLIT4, 512, 256, 576, 16),                                      # ... over 4 waves
+    (TILE128, 512, 512, 64, 16), (TILE128, 768, 768, 128, 16), (TILE128, 512, 768, 576, 13),
+    (TILE256X128, 1024, 1024, 448, 16), (TILE256X128, 1536, 1024, 64, 16), (TILE256X128, 256, 6656, 192, 16),
+    (TILE256, 1280, 1280, 1536, 16), (TILE256, 768, 768, 1088, 24),   # tiles not a multiple of 8: ranges per XCD
 ])
-def test_digits_in_small_tiles(dev, M, N, K, S):
+def test_digits_in_small_tiles(dev, tile, M, N, K, S):
+    assert hip().oz_rule_digit_tile(256, M, N, K, S) == tile
     rng = np.random.default_rng(M + 3 * N + K + S)
     A, Bt = planes(rng, S, M, K), planes(rng, S, N, K)
     desc = crt_desc(MODULI[:S], 54, 3)
@@ -44,15 +50,20 @@ def test_digits_in_small_tiles(dev, M, N, K, S):
     dev.bufs.clear()
 
 
-@pytest.mark.parametrize("M,N,K,p", [
-    (256, 256, 64, 2), (256, 256, 192, 13),                           # 32 x 32, K over 4 waves
-    (512, 512, 128, 8), (512, 256, 64, 3),                            # 64 x 64
-    (512, 512, 192, 7), (512, 256, 640, 10),                          # 64 x 64, K over 8 waves
-    (768, 1024, 512, 5), (768, 768, 576, 6), (1024, 768, 576, 7),     # all diagonals, odd and even steps
-    (768, 768, 512, 8), (768, 768, 576, 9), (2048, 1024, 2048, 8),
-    (768, 768, 448, 8), (768, 768, 576, 10), (2048, 1024, 128, 4), (1536, 2048, 384, 5),  # 128 x 128
+DIAG256, ALL, DIAG128, DIAG64, SPLIT64, SPLIT32 = range(6)
+
+
+@pytest.mark.parametrize("tile,M,N,K,p", [
+    (SPLIT32, 256, 256, 64, 2), (SPLIT32, 256, 256, 192, 13),         # 32 x 32, K over 4 waves
+    (DIAG64, 512, 512, 128, 8), (DIAG64, 512, 256, 64, 3),
+    (SPLIT64, 512, 512, 192, 7), (SPLIT64, 512, 256, 640, 10),        # 64 x 64, K over 8 waves
+    (ALL, 768, 1024, 512, 5), (ALL, 768, 768, 576, 6), (ALL, 1024, 768, 576, 7),  # odd and even steps
+    (ALL, 768, 768, 512, 8), (ALL, 768, 768, 576, 9), (ALL, 2048, 1024, 2048, 8),
+    (DIAG128, 768, 768, 448, 8), (DIAG128, 768, 768, 576, 10), (DIAG128, 2048, 1024, 128, 4), (DIAG128, 1536, 2048, 384, 5),
+    (DIAG256, 1280, 1280, 128, 11), (DIAG256, 1536, 1536, 192, 8),
 ])
-def test_diagonals_in_small_tiles(dev, M, N, K, p):
+def test_diagonals_in_small_tiles(dev, tile, M, N, K, p):
+    assert hip().oz_rule_diag_tile(256, M, N, K, p) == tile
     dmax = 127 if p * K * 127 * 127 < 2**31 else 32
     rng = np.random.default_rng(M + 3 * N + K + p)
     A, Bt = (np.clip(planes(rng, p, R, K), -dmax, dmax) for R in (M, N))
