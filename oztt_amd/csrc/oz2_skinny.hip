@@ -15,7 +15,7 @@
 //   - B's blocks (4 S KB per K block, 64 rows of planes) come into LDS once for the 8 waves, a block ahead.
 // A's residues may be any representatives (the products are reduced), so the even modulus goes the way of the
 // odd ones, whatever the planes' sequence makes of a tie, and a small modulus that of a multiple. A workgroup that met
-// an element without a place in the digits (its row has a range flag) computes its rows once more from the planes' own
+// an element without a place in the bytes (its row has a range flag) computes its rows once more from the planes' own
 // residues, so that flagged rows come out as the stages give them too.
 // Bound by the VALU work of the residues (54% busy) and, for A's 64 KB rows, by the memory channels: without the
 // reads of A the pass takes 88 us less, without B's copies 46, without the residues' VALU work 29.
@@ -48,6 +48,16 @@ struct SkinnyConsts {
     int init[kMaxS], mneg[kMaxS];
     int even;  // the even modulus of the set or -1, with the constants of its sequence on the digits (residue_f)
     float m, rinv, c0, c1;
+};
+
+// Whether any of some elements has |x 2^d| >= 2^22 or is an infinity or NaN, by the upper words of split_integer3 (the
+// integer part stands 12 bits below it). A' of the others fits its 8 bytes, |A'| < 2^63, and every residue of it is that
+// of its digits; from 2^23 on the bytes are A' modulo 2^64, which is another residue for the even modulus. The scale
+// leaves at most 2^(b - 40) <= 2^20 unless a range flag is raised for the row, wherever in the row its reason stands.
+struct BeyondBytes {
+    uint32_t top = 0;
+    __device__ __forceinline__ void add(uint32_t T) { top = max(top, T - (0x41F80000u - 0x400u)); }
+    __device__ __forceinline__ bool any() const { return top >= 0x800u; }
 };
 
 __device__ __forceinline__ int residue_byte(int u, int v, uint32_t magic, int mneg) {
@@ -118,14 +128,14 @@ __global__ void __launch_bounds__(512) skinny_kernel(const double* __restrict__ 
             }
         }
     };
-    FarElements far;  // over all elements of this thread
+    BeyondBytes far;  // over all elements of this thread
     auto convert = [&](const double* x, v4i* g) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             uint32_t a0[2], a1[2];
             float dig[3];
-            far.add(split_integer3(live ? x[2 * j] : 0.0, delta, a0, dig), 0);
-            far.add(split_integer3(live ? x[2 * j + 1] : 0.0, delta, a1, dig), 0);
+            far.add(split_integer3(live ? x[2 * j] : 0.0, delta, a0, dig));
+            far.add(split_integer3(live ? x[2 * j + 1] : 0.0, delta, a1, dig));
             g[j] = v4i{(int)a0[0], (int)a0[1], (int)a1[0], (int)a1[1]};
         }
     };
@@ -209,7 +219,7 @@ __global__ void __launch_bounds__(512) skinny_kernel(const double* __restrict__ 
     }
     wait_vmcnt_lgkm0<0>();  // the last block's copies, issued twice
     __syncthreads();
-    // Elements that are Far (an operand with a range flag) are what the procedure makes of them, also in the even
+    // Elements beyond their bytes (an operand with a range flag) are what the procedure makes of them, also in the even
     // modulus, whose sequence on the digits then is no residue of A': rows with such elements once more, their residues
     // by the functions of the planes and through LDS.
     int* seen = reinterpret_cast<int*>(states);

@@ -119,6 +119,19 @@ def test_flagged_operands_equal_the_stages(dev, M, N, K, width, moduli):
     assert way == (PREP | FUSED if M == 1500 else PREP if K <= 512 else 0 if M == 300 else PART if M > 12224 else 2 * PART)
 
 
+# One such element per row, beside values that its flag leaves larger than the scale would: their digits hold, but not in
+# the bytes that the narrow kernel makes of A' (the even modulus again). Between 2^2 and 2^20, in rows that have the flag's
+# element in the first K block, the last, and the middle one (K in two parts for the last two).
+@pytest.mark.parametrize("M,N,K", [(12290, 64, 1100), (6100, 20, 1030), (8192, 64, 2048)])
+@pytest.mark.parametrize("log2", [2, 6, 7, 8, 9, 12, 16, 20])
+def test_flagged_rows_with_large_values_equal_the_stages(dev, M, N, K, log2):
+    A, B = operands(M, N, K, M + K, 0.5)
+    rows = np.arange(9, M, 97)
+    A[rows] *= 2.0 ** log2
+    A[rows, np.array([0, K // 2, K - 1])[rows % 3]] = np.array([np.inf, 2.0 ** 130, np.nan])[rows % 3]
+    assert pass_equals_stages(dev, A, B, M, N, K, 0, operands(M, N, K, 1, 0.5)) // PART in (1, 2)
+
+
 def pass_equals_stages(dev, A, B, M, N, K, width, plan=None, want_flags=None, moduli=None):
     # width 0: the plan; up to 60 bits: the plan at that width; above: the moduli for it, in four or five digits (the
     # planner stops at 16 moduli)
