@@ -15,8 +15,8 @@
 //   - B's blocks (4 S KB per K block, 64 rows of planes) come into LDS once for the 8 waves, a block ahead.
 // A's residues may be any representatives (the products are reduced), so the even modulus goes the way of the
 // odd ones, whatever the planes' sequence makes of a tie, and a small modulus that of a multiple. A workgroup that met
-// an element without a place in the bytes (its row has a range flag) computes its rows once more from the planes' own
-// residues, so that flagged rows come out as the stages give them too.
+// an element without a place in the bytes (its row has a range flag) puts the planes' own residues in its place at the
+// end, so that flagged rows come out as the stages give them too.
 // Bound by the VALU work of the residues (54% busy) and, for A's 64 KB rows, by the memory channels: without the
 // reads of A the pass takes 88 us less, without B's copies 46, without the residues' VALU work 29.
 // Whole pass, us, with planes -> here: 8192 x 64 x 8192: 645 -> 405; 8192 x 1 x 8192: 632 -> 413; 12288 x 64 x
@@ -220,8 +220,11 @@ __global__ void __launch_bounds__(512) skinny_kernel(const double* __restrict__ 
     wait_vmcnt_lgkm0<0>();  // the last block's copies, issued twice
     __syncthreads();
     // Elements beyond their bytes (an operand with a range flag) are what the procedure makes of them, also in the even
-    // modulus, whose sequence on the digits then is no residue of A': rows with such elements once more, their residues
-    // by the functions of the planes and through LDS.
+    // modulus, whose sequence on the digits then is no residue of A'. A workgroup that met any goes over its elements
+    // again, and in the K blocks that hold some it takes these elements' products back out of the sums and puts in
+    // those of the planes' residues: of A' the same byte as above, by the same steps (every product is exact modulo
+    // 2^32, so only the sums that stand at the end have to fit). 6272 x 64 x 1536, 16 moduli, three such elements:
+    // 149 us (108 without any; 320 with every block of these rows computed again; 140 by the planes).
     int* seen = reinterpret_cast<int*>(states);
     if (lane == 0) seen[wave] = 0;
     if (far.any() || delta >= 541) seen[wave] = 1;
@@ -230,22 +233,57 @@ __global__ void __launch_bounds__(512) skinny_kernel(const double* __restrict__ 
 #pragma unroll
     for (int i = 0; i < 8; i++) again |= seen[i] != 0;
     if (__builtin_expect(again, 0)) {
-#pragma unroll
-        for (int i = 0; i < 2 * P; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[i][j] = v4i{0, 0, 0, 0};
+        // (the sums leave few registers: the lane's place is taken afresh)
+        int t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        const int lane = t & 63, lrow = t >> 3, lq = t & 7, row = min(row0 + lrow, M - 1);
+        const bool live = row0 + lrow < M;
+        const int32_t delta = dA[row];
+        const int foff = fragment16_offset(lane);
         for (int i = 0; i < steps; i++) {
-            load(x, st0 + i);
-            __syncthreads();
+            auto element = [&](int e) {
+                const int kk = (st0 + i) * 64 + 2 * lq + 16 * (e >> 1) + (e & 1);
+                const double v = A[(size_t)row * lda + min(kk, K - 1)];
+                return live && kk < K ? v : 0.0;
+            };
+            uint32_t mine = 0;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 uint32_t a[2];
                 float dig[3];
-                make_digits<3>(live ? x[e] : 0.0, delta, dig);
+                BeyondBytes f;
+                f.add(split_integer3(element(e), delta, a, dig));
+                mine |= (f.any() || delta >= 541 ? 1u : 0u) << e;
+            }
+            // the votes of two blocks in turn: those of this one are read before the next barrier
+            int* vote = seen + 8 + 8 * (i & 1);
+            const bool any = __ballot(mine != 0) != 0;
+            if (lane == 0) vote[wave] = any;
+            __syncthreads();
+            int votes = 0;
+#pragma unroll
+            for (int w = 0; w < 8; w++) votes |= vote[w];
+            if (!__builtin_amdgcn_readfirstlane(votes)) continue;
+            for (int q = t; q < 256 * S; q += 512) {
+                reinterpret_cast<v4i*>(lds)[q] = v4i{0, 0, 0, 0};
+                reinterpret_cast<v4i*>(lds + kBuf)[q] = v4i{0, 0, 0, 0};
+            }
+            __syncthreads();
+            for (; mine; mine &= mine - 1) {
+                const int e = __builtin_ctz(mine);
+                const double v = element(e);
+                uint32_t taken[2], a[2];
+                float dig[3];
+                split_integer3(v, delta, taken, dig);
+                make_digits<3>(v, delta, dig);
                 balanced_bytes<3>(dig, a);
                 int8_t* at = lds + 64 * lrow + 2 * lq + 16 * (e >> 1) + (e & 1);
                 for (int s = 0; s < S; s++) {
+                    const int dot = __builtin_amdgcn_sdot4((int)taken[1], (int)k.w[s][1],
+                                                           __builtin_amdgcn_sdot4((int)taken[0], (int)k.w[s][0], 0, false), false);
+                    const int u = dot + k.init[s];
                     const float m = (float)((1 << 24) - k.mneg[s]);
+                    at[kBuf + 4096 * s] = (int8_t)residue_byte(u, u + dot, k.magic[s], k.mneg[s]);
                     at[4096 * s] = (int8_t)(int)(s == k.even ? residue_f<3>(dig, k.m, k.rinv, k.c0, k.c1, 0.0f, 0.0f)
                                                              : residue_odd<2>(a, k.w[s], m, 1.0f / m));
                 }
@@ -254,12 +292,14 @@ __global__ void __launch_bounds__(512) skinny_kernel(const double* __restrict__ 
 #pragma unroll
             for (int g = 0; g < 2 * P; g++) {
                 const int s = min(s0 + g, S - 1);
-                const v4i f = *reinterpret_cast<const v4i*>(lds + 4096 * s + 64 * (16 * band + r) + 16 * c);
+                const int8_t* at = lds + 4096 * s + 64 * (16 * band + (lane & 15)) + 16 * (lane >> 4);
+                const v4i in = *reinterpret_cast<const v4i*>(at), out = *reinterpret_cast<const v4i*>(at + kBuf);
 #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    acc[g][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                        f, *reinterpret_cast<const v4i*>(pB + ((long long)s * sB + ((long long)j * nk + st0 + i) * 1024 + foff)),
-                        acc[g][j], 0, 0, 0);
+                for (int j = 0; j < 4; j++) {
+                    const v4i b = *reinterpret_cast<const v4i*>(pB + ((long long)s * sB + ((long long)j * nk + st0 + i) * 1024 + foff));
+                    const v4i less = __builtin_amdgcn_mfma_i32_16x16x64_i8(out, b, -acc[g][j], 0, 0, 0);
+                    acc[g][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(in, b, -less, 0, 0, 0);
+                }
             }
         }
         __syncthreads();

@@ -114,7 +114,7 @@ def test_flagged_operands_equal_the_stages(dev, M, N, K, width, moduli):
         X[12] *= np.exp2(rng.integers(-60, 1000, n))
         X[13] = 2.0 ** -1060
         X[15, n - 1] = 2.0 ** 128
-    A[M - 1, K - 1] = np.nan
+    A[M - 1, K - 1], A[M // 2, K // 2] = np.nan, -np.inf  # by themselves in their rows and K blocks
     way = pass_equals_stages(dev, A, B, M, N, K, width, operands(M, N, K, 1, 0.5), moduli=moduli)
     assert way == (PREP | FUSED if M == 1500 else PREP if K <= 512 else 0 if M == 300 else PART if M > 12224 else 2 * PART)
 
