@@ -191,10 +191,12 @@ int oz2_crt_digits_f64(oz_dev* dev, const uint8_t* D, int M, int N, int ldd, lon
 /* ---- A5-A11 in one call: the whole Scheme II INT8 pass on device-resident operands ----------
  * (reference ozaki2.cpp:439-478: scale, slice, products, reconstruction; the plan is the caller's,
  * made on the host as for the C++ backend.) C (M x N, leading dimension ldc) = A B for row-major A
- * (M x K, lda) and B (K x N, ldb): flags[0..1] <- 0; oz_scale_f64 (ceil mode 1, shift crt->shift)
- * of A's rows and B's columns, ORing their range flags into flags[0] and flags[1] (as
+ * (M x K, lda) and B (K x N, ldb), with the result of these stages: oz_scale_f64 (ceil mode 1, shift crt->shift)
+ * of A's rows and B's columns, whose range flags go to flags[0] and flags[1] (as
  * oz_scale_f64: 1, 2, 4; the caller reads them); oz2_split_int8 of A (layout 2) and B (layout 3);
- * oz2_gemm_digits; oz2_crt_digits_f64. Every launch is ordered on the handle's stream; nothing
+ * oz2_gemm_digits; oz2_crt_digits_f64. The two flag words need no clearing: the last launch writes both, and
+ * so does a pass that a stage refuses on its way (what the scale had found by then); a call that is refused
+ * before its first launch (OZ_ERR_ARG for pointers, extents, plan or workspace) leaves them. Every launch is ordered on the handle's stream; nothing
  * waits on the host. mo and crt must hold the same INT8 moduli, crt->shift = crt->b - 20 (mo->nd - 1),
  * and K (rounded up to 64) times 127^2 must stay below 2^31. flags: two device words, 4-byte aligned.
  * The intermediates live in `work` (256-byte aligned): the exponent deltas, the S residue planes of

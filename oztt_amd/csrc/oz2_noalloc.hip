@@ -7,8 +7,8 @@
 // In host code the array's name is only a stand-in, not a device address. Its address on a GPU is
 // looked up once per device, with that device current (hipGetSymbolAddress), kept in `scratch_ptr`,
 // and only that address is ever handed to a kernel. Every call on one GPU shares that GPU's array,
-// which keeps the previous call's contents; the pass clears what must start at zero (the range
-// flags) with a fill kernel and writes every other region in full before reading it. Calls that
+// which keeps the previous call's contents; the pass writes every region that it reads in full before (the
+// range flags are gathered in words of the handle, which are zero between passes). Calls that
 // overlap on one GPU (two handles' streams, or two host threads) race for the array.
 #include <mutex>
 

@@ -1,11 +1,15 @@
 // Scheme II INT8, the whole device pass in one call: for device-resident FP64 operands and a plan
-// made on the host (the moduli and CRT descriptors of include/oz_hip.h), C = A B through the same
-// stage kernels the C++ backend issues one by one (reference ozaki2.cpp:439-478: scale, slice,
-// products, reconstruction):
+// made on the host (the moduli and CRT descriptors of include/oz_hip.h), C = A B as the stages give it
+// (reference ozaki2.cpp:439-478: scale, slice, products, reconstruction):
 //   row maxima of A and column maxima of B -> exponent deltas and range flags (oz_scale_pair_f64);
 //   residue planes of A and of B^T in OZ_BLOCK tiles (oz2_split_pair_int8);
 //   products reduced to CRT digits in the GEMM epilogue (oz2_gemm_digits);
 //   exact CRT to FP64 (oz2_crt_digits_f64).
+// These four launches are the general route. By sizes and moduli (route_of) some of them become one, with the
+// same C and flags bit for bit, rows and columns with a range flag included:
+//   short K: the first two (oz2_prep.hip);
+//   short K and many tiles: the last two (oz2_gemm_crt.hip), with either form of the first two;
+//   at most 64 columns and long K: A's planes are never made (oz2_skinny.hip), B's come from the stage.
 // Every launch is ordered on the handle's stream and nothing waits on the host, so a caller that
 // keeps its operands on the GPU can queue many passes back to back.
 //

@@ -1,6 +1,8 @@
 """The residue generator's A' for nd = 3 (split_integer3 in oztt_amd/csrc/oz2_residue.hpp), which follows the
 reference's binary32 digit procedure through binary64 operations, against that procedure itself (load_triple
-and make_digits in oz_tf32.hpp / oz2_residue.hpp, restated here operation by operation in float32). CPU only."""
+and make_digits in oz_tf32.hpp / oz2_residue.hpp, restated here operation by operation in float32). CPU only:
+both sides are restatements, so this shows that the one sequence equals the other; that the kernels hold them is what
+tests/test_gpu_stages.py (against the oracle) and tests/test_gpu_far_elements.py show."""
 import numpy as np
 
 F = np.float32
