@@ -69,7 +69,8 @@ __device__ __forceinline__ void store_digits16(const int32_t* src, uint8_t* dst,
 // coalesced 1 KB load each. Bound by those loads (a tile of 64 x 64 reads 8 KB for 16 MFMAs, about half
 // of what the matrix cores could take from L2), so it serves where the 256 x 256 tiles (or, for the
 // diagonals, the all-diagonals kernel's 64 x 64) are too few for the chip. 256 x 256 x 32768, 16 moduli
-// (256 tiles): 255.6 -> 50.6 us launch after launch, 290 -> 78 in a pass (the planes in no cache yet); 256 x 256 x 2048, 8 diagonals: 141 -> 16.5 us.
+// (256 tiles): 255.6 -> 50.6 us launch after launch, 290 -> 78 in a pass (the planes in no cache yet);
+// 256 x 256 x 2048, 8 diagonals: 141 -> 16.5 us.
 template <int MODE, int TI, int TJ, int KW, int P>
 __global__ void __launch_bounds__(64 * KW) gemm_i8_ksplit_kernel(const int8_t* __restrict__ A,
                                                                  const int8_t* __restrict__ Bt, void* __restrict__ C,
